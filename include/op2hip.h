@@ -188,6 +188,15 @@ int op2hip_transpose_fill(int32_t nrows, const int32_t *map, int32_t arity,
                           int32_t iter_size, const int32_t *inc_ptr,
                           int32_t *inc_ent, void *work, size_t work_bytes,
                           void *stream);
+/* The same with `places` (device, iter_size * arity int32, written by count):
+ * each entry's place among its row's, so that fill needs no atomics. */
+int op2hip_transpose_count_places(int32_t nrows, const int32_t *map, int32_t arity,
+                                  int32_t iter_size, int32_t *inc_ptr,
+                                  int64_t *total_host, int32_t *places, void *work,
+                                  size_t work_bytes, void *stream);
+int op2hip_transpose_fill_places(int32_t nrows, const int32_t *map, int32_t arity,
+                                 int32_t iter_size, const int32_t *inc_ptr,
+                                 const int32_t *places, int32_t *inc_ent, void *stream);
 
 /* ---- sparsity (replaces pyop2/sparsity.pyx:121-284, build_sparsity and
  *      fill_with_zeros, non-extruded, one DataSet pair) ------------------ */

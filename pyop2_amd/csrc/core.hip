@@ -142,15 +142,30 @@ static int scan(int64_t n, const int32_t *in, int32_t *out, int64_t *total_host,
 // ---------------------------------------------------------------------------
 // map transpose
 
+// pos (may be null): each entry's place among its row's entries, as counted.
 __global__ void transpose_count(int32_t nrows, const int32_t *__restrict__ map,
                                 int64_t nent, int32_t *__restrict__ counts,
-                                int32_t *__restrict__ bad) {
+                                int32_t *__restrict__ bad, int32_t *__restrict__ pos) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nent;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int32_t r = map[i];
     if (r < 0) continue;
     if (r >= nrows) { atomicAdd(bad, 1); continue; }
-    atomicAdd(&counts[r], 1);
+    const int32_t at = atomicAdd(&counts[r], 1);
+    if (pos) pos[i] = at;
+  }
+}
+
+// With the places found while counting, filling needs no second round of
+// atomics (48 us for the P2 24^3 cube's 829,440 entries, 9 us with them);
+// without, each row's cursor hands them out.
+__global__ void transpose_place(int32_t nrows, const int32_t *__restrict__ map, int64_t nent,
+                                const int32_t *__restrict__ inc_ptr,
+                                const int32_t *__restrict__ pos, int32_t *__restrict__ inc_ent) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nent;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t r = map[i];
+    if (r >= 0 && r < nrows) inc_ent[(int64_t)inc_ptr[r] + pos[i]] = static_cast<int32_t>(i);
   }
 }
 
@@ -166,22 +181,62 @@ __global__ void transpose_fill(int32_t nrows, const int32_t *__restrict__ map,
   }
 }
 
-// Sort each row's incidence list ascending (lists are short: one thread each).
-__global__ void transpose_sort(int32_t nrows, const int32_t *__restrict__ inc_ptr,
-                               int32_t *__restrict__ inc_ent) {
-  for (int32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < nrows;
-       r += gridDim.x * blockDim.x) {
-    const int32_t lo = inc_ptr[r], hi = inc_ptr[r + 1];
-    for (int32_t a = lo + 1; a < hi; ++a) {
-      const int32_t v = inc_ent[a];
-      int32_t b = a - 1;
-      while (b >= lo && inc_ent[b] > v) {
-        inc_ent[b + 1] = inc_ent[b];
-        --b;
+// Sort each row's incidence list ascending.  A block takes 256 rows and stages
+// their lists in LDS; every entry then finds its place by counting the smaller
+// entries of its row, all entries of the block at once (one thread sorting a
+// row in memory is a chain of dependent loads: 52 us for the 82,944 cells and
+// 117,649 nodes of the P2 24^3 cube, 20 us this way).  Rows whose lists do not
+// fit the stage together are sorted by one thread each.
+constexpr int kSortRows = 256;
+constexpr int kSortStage = 7168;
+
+__global__ void __launch_bounds__(kSortRows)
+transpose_sort(int32_t nrows, const int32_t *__restrict__ inc_ptr,
+               int32_t *__restrict__ inc_ent) {
+  __shared__ int32_t ptr[kSortRows + 1];
+  __shared__ int32_t ent[kSortStage];
+  for (int64_t r0 = (int64_t)blockIdx.x * kSortRows; r0 < nrows;
+       r0 += (int64_t)gridDim.x * kSortRows) {
+    const int32_t nr = (int32_t)min((int64_t)kSortRows, nrows - r0);
+    for (int32_t k = threadIdx.x; k <= nr; k += kSortRows) ptr[k] = inc_ptr[r0 + k];
+    __syncthreads();
+    const int32_t base = ptr[0], n = ptr[nr] - base;
+    if (n <= kSortStage) {
+      for (int32_t k = threadIdx.x; k < n; k += kSortRows) ent[k] = inc_ent[(int64_t)base + k];
+      __syncthreads();
+      for (int32_t k = threadIdx.x; k < n; k += kSortRows) {
+        int32_t a = 0, b = nr;   // the row of entry k: the last one that starts at or before it
+        while (b - a > 1) {
+          const int32_t mid = (a + b) >> 1;
+          if (ptr[mid] - base <= k) a = mid; else b = mid;
+        }
+        const int32_t lo = ptr[a] - base, hi = ptr[a + 1] - base, v = ent[k];
+        int32_t rank = 0;
+        for (int32_t t = lo; t < hi; ++t) rank += ent[t] < v;
+        inc_ent[(int64_t)base + lo + rank] = v;
       }
-      inc_ent[b + 1] = v;
+    } else if ((int32_t)threadIdx.x < nr) {
+      const int32_t lo = ptr[threadIdx.x], hi = ptr[threadIdx.x + 1];
+      for (int32_t a = lo + 1; a < hi; ++a) {
+        const int32_t v = inc_ent[a];
+        int32_t b = a - 1;
+        while (b >= lo && inc_ent[b] > v) {
+          inc_ent[b + 1] = inc_ent[b];
+          --b;
+        }
+        inc_ent[b + 1] = v;
+      }
     }
+    __syncthreads();  // the next rows reuse the stage
   }
+}
+
+static int sort_incidences(int32_t nrows, const int32_t *inc_ptr, int32_t *inc_ent, hipStream_t s) {
+  if (nrows <= 0) return OP2HIP_OK;
+  transpose_sort<<<std::min<uint32_t>(ceil_div(nrows, kSortRows), 16384), kSortRows, 0, s>>>(
+      nrows, inc_ptr, inc_ent);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
 }
 
 static size_t transpose_bytes(int32_t nrows) {
@@ -191,7 +246,7 @@ static size_t transpose_bytes(int32_t nrows) {
 }
 
 // ---------------------------------------------------------------------------
-// sparsity rows: one 64-thread block per block row
+// sparsity rows: the sorted distinct columns of every block row
 
 struct PairTable {
   const int32_t *cmap[OP2HIP_MAX_PAIRS];
@@ -245,26 +300,177 @@ __device__ __forceinline__ int32_t block64_min(int32_t v, int32_t *lds) {
   return s;
 }
 
-template <bool kFill>
-__global__ void __launch_bounds__(64)
+// Rows of at most kCap candidates: a group of kLanes lanes takes a row, reads
+// its candidates (at most six a lane, all loads issued together) and enters
+// them in the group's hash table in LDS; a lane whose entry was new holds one
+// distinct column.  Counting is then the number of new entries, and filling
+// ranks every distinct column among the others.  Comparing all pairs of
+// candidates took 412 us (count) and 873 us (fill) for the 117,649 rows of the
+// P2 24^3 cube, whose candidates (50 an edge, 240 a vertex) repeat 2 to 4
+// times; a table visit per candidate takes 51 and 94 us.
+template <int kLanes>
+struct RowTable {
+  static constexpr int kSlots = kLanes * 8;     // a power of two
+  static constexpr int kRounds = 6;
+  static constexpr int kCap = kLanes * kRounds; // three quarters of the slots
+  static constexpr int kGroups = 256 / kLanes;
+};
+
+// LDS accesses before it are seen by those after it in every lane of the wave.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ int64_t row_candidates(const PairTable &pt, int32_t r, int32_t ncols,
+                                                  int32_t set_diag) {
+  int64_t m = set_diag && r < ncols ? 1 : 0;
+  for (int p = 0; p < pt.npairs; ++p)
+    m += (int64_t)(pt.inc_ptr[p][r + 1] - pt.inc_ptr[p][r]) * pt.carity[p];
+  return m;
+}
+
+template <bool kFill, int kLanes>
+__global__ void __launch_bounds__(256)
 sparsity_rows(int32_t nrows, int32_t ncols, PairTable pt, int32_t set_diag,
               const int32_t *__restrict__ rowptr, int32_t *__restrict__ out) {
+  using Tab = RowTable<kLanes>;
+  constexpr int kR = Tab::kRounds;
+  __shared__ int32_t tables[Tab::kGroups][Tab::kSlots];
+  __shared__ __align__(16) int32_t uniques[kFill ? Tab::kGroups : 1][kFill ? Tab::kCap : 1];
+  __shared__ int32_t lo[Tab::kGroups][OP2HIP_MAX_PAIRS], cnt[Tab::kGroups][OP2HIP_MAX_PAIRS];
+  const int grp = threadIdx.x / kLanes, lane = threadIdx.x % kLanes;
+  const int shift = (threadIdx.x & 63) / kLanes * kLanes;   // of the group's bits in a ballot
+  const uint64_t group_mask = kLanes == 64 ? ~0ull : ((1ull << (kLanes & 63)) - 1);
+  int32_t *table = tables[grp];
+  for (int k = lane; k < Tab::kSlots; k += kLanes) table[k] = -1;
+  const int64_t step = (int64_t)gridDim.x * Tab::kGroups;
+  int32_t first_inc = 0, ninc = 0;   // of the next row, one pair a lane
+  auto load_range = [&](int64_t r) {
+    if (lane < pt.npairs && r < nrows) {
+      first_inc = pt.inc_ptr[lane][r];
+      ninc = pt.inc_ptr[lane][r + 1] - first_inc;
+    }
+  };
+  load_range((int64_t)blockIdx.x * Tab::kGroups + grp);
+  for (int64_t r0 = (int64_t)blockIdx.x * Tab::kGroups + grp; r0 < nrows; r0 += step) {
+    const int32_t r = (int32_t)r0;
+    wave_lds_sync();   // the previous row is done with them
+    if (lane < pt.npairs) {
+      lo[grp][lane] = first_inc;
+      cnt[grp][lane] = ninc;
+    }
+    wave_lds_sync();
+    load_range(r0 + step);
+    const int32_t base = kFill ? rowptr[r] : 0;
+    const bool has_diag = set_diag && r < ncols;
+    int64_t total = has_diag ? 1 : 0;
+    for (int p = 0; p < pt.npairs; ++p) total += (int64_t)cnt[grp][p] * pt.carity[p];
+    if (total > Tab::kCap) continue;   // sparsity_long_rows takes it
+    const int m = (int)total;
+    // every lane's incidences, then every lane's columns
+    int32_t c[kR], slot[kR], col[kR], pair[kR];
+#pragma unroll
+    for (int u = 0; u < kR; ++u) {
+      if (u * kLanes >= m) break;
+      uint32_t k = lane + u * kLanes;
+      c[u] = pair[u] = -1;
+      if (k >= (uint32_t)m) continue;
+      for (int p = 0; p < pt.npairs; ++p) {
+        const uint32_t ar = (uint32_t)pt.carity[p], n = (uint32_t)cnt[grp][p] * ar;
+        if (k < n) {
+          const uint32_t q = k / ar;
+          pair[u] = p;
+          col[u] = (int32_t)(k - q * ar);
+          c[u] = pt.inc_ent[p][lo[grp][p] + (int32_t)q];
+          break;
+        }
+        k -= n;
+      }
+      if (pair[u] < 0) c[u] = r;   // past the pairs' candidates: the diagonal
+    }
+#pragma unroll
+    for (int u = 0; u < kR; ++u) {
+      if (u * kLanes >= m) break;
+      if (pair[u] < 0) continue;
+      const int p = pair[u];
+      const int32_t e = (int32_t)((uint32_t)c[u] / (uint32_t)pt.rarity[p]);
+      c[u] = pt.cmap[p][(int64_t)e * pt.carity[p] + col[u]];
+    }
+    int count = 0;
+#pragma unroll
+    for (int u = 0; u < kR; ++u) {
+      if (u * kLanes >= m) break;
+      slot[u] = -1;
+      if (c[u] >= 0) {
+        uint32_t h = ((uint32_t)c[u] * 2654435761u) / (uint32_t)(0x100000000ull / Tab::kSlots);
+        for (;;) {   // ends: fewer entries than slots
+          const int32_t was = atomicCAS(&table[h], -1, c[u]);
+          if (was == -1) slot[u] = (int32_t)h;
+          if (was == -1 || was == c[u]) break;
+          h = (h + 1) & (Tab::kSlots - 1);
+        }
+      }
+      const uint64_t news = (__ballot(slot[u] >= 0) >> shift) & group_mask;
+      if constexpr (kFill) {
+        if (slot[u] >= 0) uniques[grp][count + __popcll(news & ((1ull << lane) - 1))] = c[u];
+      }
+      count += __popcll(news);
+    }
+    if constexpr (!kFill) {
+      if (lane == 0) out[r] = count;
+    } else {
+      if (lane < 3 && count + lane < Tab::kCap) uniques[grp][count + lane] = INT32_MAX;
+      wave_lds_sync();
+      const int4 *quad = reinterpret_cast<const int4 *>(uniques[grp]);
+      int32_t *row = out + base;
+#pragma unroll
+      for (int u = 0; u < kR; ++u) {
+        if (u * kLanes >= m) break;
+        if (slot[u] < 0) continue;
+        int rank = 0;
+        for (int t = 0; t < (count + 3) / 4; ++t) {
+          const int4 q = quad[t];
+          rank += (q.x < c[u]) + (q.y < c[u]) + (q.z < c[u]) + (q.w < c[u]);
+        }
+        row[rank] = c[u];
+      }
+    }
+    // the slots this lane filled are emptied for the next row
+#pragma unroll
+    for (int u = 0; u < kR; ++u) {
+      if (u * kLanes >= m) break;
+      if (slot[u] >= 0) table[slot[u]] = -1;
+    }
+    wave_lds_sync();
+  }
+}
+
+// Rows of more than `cap` candidates, a block of 64 threads for 64 rows in
+// turn: all pairs of candidates up to kRowCap, repeated minimum extraction
+// straight from the maps beyond.
+template <bool kFill>
+__global__ void __launch_bounds__(64)
+sparsity_long_rows(int32_t nrows, int32_t ncols, PairTable pt, int32_t set_diag, int32_t cap,
+                   const int32_t *__restrict__ rowptr, int32_t *__restrict__ out) {
   __shared__ int32_t cand[kRowCap];
   __shared__ uint8_t first[kRowCap];
   __shared__ int32_t red[64];
   __shared__ int32_t lo[OP2HIP_MAX_PAIRS], cnt[OP2HIP_MAX_PAIRS];
-  for (int32_t r = blockIdx.x; r < nrows; r += gridDim.x) {
+  const int64_t r0 = (int64_t)blockIdx.x * 64, mine_r = r0 + threadIdx.x;
+  uint64_t todo = __ballot(mine_r < nrows && row_candidates(pt, (int32_t)mine_r, ncols, set_diag) > cap);
+  for (; todo; todo &= todo - 1) {
+    const int32_t r = (int32_t)(r0 + __ffsll((unsigned long long)todo) - 1);
     if (threadIdx.x < (unsigned)pt.npairs) {
       const int p = threadIdx.x;
       lo[p] = pt.inc_ptr[p][r];
       cnt[p] = pt.inc_ptr[p][r + 1] - lo[p];
     }
     __syncthreads();
-    int64_t m = 0;
-    for (int p = 0; p < pt.npairs; ++p) m += (int64_t)cnt[p] * pt.carity[p];
     const bool has_diag = set_diag && r < ncols;
     const int32_t diag_col = has_diag ? r : -1;
-    m += has_diag ? 1 : 0;
+    const int64_t m = row_candidates(pt, r, ncols, set_diag);
     const int32_t base = kFill ? rowptr[r] : 0;
     if (m <= kRowCap) {
       for (int64_t k = threadIdx.x; k < m; k += 64)
@@ -293,7 +499,7 @@ sparsity_rows(int32_t nrows, int32_t ncols, PairTable pt, int32_t set_diag,
       }
       __syncthreads();
     } else {
-      // long row: repeated minimum extraction straight from the maps
+      // longer still: repeated minimum extraction straight from the maps
       int32_t last = -1, count = 0;
       for (;;) {
         int32_t best = INT32_MAX;
@@ -311,6 +517,37 @@ sparsity_rows(int32_t nrows, int32_t ncols, PairTable pt, int32_t set_diag,
       __syncthreads();
     }
   }
+}
+
+// Blocks of a launch over rows.  Counting: as many as the chip holds at once,
+// so that a block empties its tables once and reads its next row's range ahead
+// (51 us against 57 for the P2 24^3 cube); filling takes longer for the rows of
+// vertices, and one row a group shares them out better (94 against 112 us).
+template <bool kFill>
+constexpr uint32_t kRowBlocks = kFill ? 65536 : 2048;
+
+// Half a wave takes rows of up to 32 candidates on average (P1 triangles: 19),
+// a whole wave longer ones (P2 tetrahedra: 73).
+template <bool kFill>
+static int launch_sparsity_rows(int32_t nrows, int32_t ncols, const op2hip_map_pair *pairs,
+                                const PairTable &pt, int32_t set_diag, const int32_t *rowptr,
+                                int32_t *out, hipStream_t s) {
+  if (nrows <= 0) return OP2HIP_OK;
+  double cands = set_diag ? nrows : 0;
+  for (int p = 0; p < pt.npairs; ++p)
+    cands += (double)pairs[p].iter_size * pt.rarity[p] * pt.carity[p];
+  const bool half = cands <= 32.0 * nrows;
+  if (half)
+    sparsity_rows<kFill, 32><<<std::min<uint32_t>(ceil_div(nrows, RowTable<32>::kGroups), kRowBlocks<kFill>),
+                               256, 0, s>>>(nrows, ncols, pt, set_diag, rowptr, out);
+  else
+    sparsity_rows<kFill, 64><<<std::min<uint32_t>(ceil_div(nrows, RowTable<64>::kGroups), kRowBlocks<kFill>),
+                               256, 0, s>>>(nrows, ncols, pt, set_diag, rowptr, out);
+  OP2HIP_LAUNCHED();
+  sparsity_long_rows<kFill><<<ceil_div(nrows, 64), 64, 0, s>>>(
+      nrows, ncols, pt, set_diag, half ? RowTable<32>::kCap : RowTable<64>::kCap, rowptr, out);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
 }
 
 __global__ void expand_rowptr(int32_t nrows, const int32_t *__restrict__ rowptr,
@@ -406,9 +643,9 @@ int op2hip_transpose_workspace(int32_t nrows, size_t *bytes) {
   return OP2HIP_OK;
 }
 
-int op2hip_transpose_count(int32_t nrows, const int32_t *map, int32_t arity,
-                           int32_t iter_size, int32_t *inc_ptr, int64_t *total_host,
-                           void *work, size_t work_bytes, void *stream) {
+int op2hip_transpose_count_places(int32_t nrows, const int32_t *map, int32_t arity,
+                                  int32_t iter_size, int32_t *inc_ptr, int64_t *total_host,
+                                  int32_t *places, void *work, size_t work_bytes, void *stream) {
   hipStream_t s = stream_of(stream);
   OP2HIP_REQUIRE(nrows >= 0 && arity > 0 && iter_size >= 0 && inc_ptr,
                  "transpose_count: bad arguments");
@@ -428,7 +665,7 @@ int op2hip_transpose_count(int32_t nrows, const int32_t *map, int32_t arity,
   const int64_t nent = (int64_t)iter_size * arity;
   if (nent > 0) {
     transpose_count<<<std::min<uint32_t>(ceil_div(nent, 256), 16384), 256, 0, s>>>(
-        nrows, map, nent, counts, bad);
+        nrows, map, nent, counts, bad, places);
     OP2HIP_LAUNCHED();
   }
   if ((rc = scan(nrows, counts, inc_ptr, total_host, scan_work, work_bytes - a - 256, s)))
@@ -441,6 +678,28 @@ int op2hip_transpose_count(int32_t nrows, const int32_t *map, int32_t arity,
     return OP2HIP_ERR_ARG;
   }
   return OP2HIP_OK;
+}
+
+int op2hip_transpose_count(int32_t nrows, const int32_t *map, int32_t arity,
+                           int32_t iter_size, int32_t *inc_ptr, int64_t *total_host,
+                           void *work, size_t work_bytes, void *stream) {
+  return op2hip_transpose_count_places(nrows, map, arity, iter_size, inc_ptr, total_host, nullptr,
+                                       work, work_bytes, stream);
+}
+
+int op2hip_transpose_fill_places(int32_t nrows, const int32_t *map, int32_t arity,
+                                 int32_t iter_size, const int32_t *inc_ptr,
+                                 const int32_t *places, int32_t *inc_ent, void *stream) {
+  hipStream_t s = stream_of(stream);
+  const int64_t nent = (int64_t)iter_size * arity;
+  OP2HIP_REQUIRE(nrows >= 0 && arity > 0 && iter_size >= 0 && inc_ptr && (nent == 0 || places),
+                 "transpose_fill_places: bad arguments");
+  if (nent > 0) {
+    transpose_place<<<std::min<uint32_t>(ceil_div(nent, 256), 16384), 256, 0, s>>>(
+        nrows, map, nent, inc_ptr, places, inc_ent);
+    OP2HIP_LAUNCHED();
+  }
+  return sort_incidences(nrows, inc_ptr, inc_ent, s);
 }
 
 int op2hip_transpose_fill(int32_t nrows, const int32_t *map, int32_t arity,
@@ -463,12 +722,7 @@ int op2hip_transpose_fill(int32_t nrows, const int32_t *map, int32_t arity,
         nrows, map, nent, cursor, inc_ent);
     OP2HIP_LAUNCHED();
   }
-  if (nrows > 0) {
-    transpose_sort<<<std::min<uint32_t>(ceil_div(nrows, 256), 16384), 256, 0, s>>>(
-        nrows, inc_ptr, inc_ent);
-    OP2HIP_LAUNCHED();
-  }
-  return OP2HIP_OK;
+  return sort_incidences(nrows, inc_ptr, inc_ent, s);
 }
 
 int op2hip_sparsity_count(int32_t nrows, int32_t ncols, const op2hip_map_pair *pairs,
@@ -487,11 +741,8 @@ int op2hip_sparsity_count(int32_t nrows, int32_t ncols, const op2hip_map_pair *p
     return OP2HIP_ERR_WORKSPACE;
   }
   int32_t *counts = static_cast<int32_t *>(work);
-  if (nrows > 0) {
-    sparsity_rows<false><<<std::min<int32_t>(nrows, 65536), 64, 0, s>>>(
-        nrows, ncols, pt, set_diag, nullptr, counts);
-    OP2HIP_LAUNCHED();
-  }
+  if ((rc = launch_sparsity_rows<false>(nrows, ncols, pairs, pt, set_diag, nullptr, counts, s)))
+    return rc;
   return scan(nrows, counts, rowptr, nnz_host, static_cast<char *>(work) + a,
               work_bytes - a, s);
 }
@@ -505,12 +756,7 @@ int op2hip_sparsity_fill(int32_t nrows, int32_t ncols, const op2hip_map_pair *pa
   PairTable pt;
   int rc;
   if ((rc = make_pairs(pairs, npairs, inc_ptr, inc_ent, &pt))) return rc;
-  if (nrows > 0) {
-    sparsity_rows<true><<<std::min<int32_t>(nrows, 65536), 64, 0, s>>>(
-        nrows, ncols, pt, set_diag, rowptr, colidx);
-    OP2HIP_LAUNCHED();
-  }
-  return OP2HIP_OK;
+  return launch_sparsity_rows<true>(nrows, ncols, pairs, pt, set_diag, rowptr, colidx, s);
 }
 
 int op2hip_pattern_expand(int32_t nrows, const int32_t *rowptr, const int32_t *colidx,

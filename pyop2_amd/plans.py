@@ -34,16 +34,16 @@ def transpose(m, nrows, iter_size):
     need = ctypes.c_size_t()
     dev.check(L.op2hip_transpose_workspace(nrows, ctypes.byref(need)), "transpose_workspace")
     work = dev.workspace(need.value)
+    places = dev.empty((max(m.arity * iter_size, 1),), np.int32)
     inc_ptr = dev.empty((nrows + 1,), np.int32)
     total = ctypes.c_int64()
     mv = m.device_values
-    dev.check(L.op2hip_transpose_count(nrows, dev.ptr(mv), m.arity, iter_size, dev.ptr(inc_ptr),
-                                       ctypes.byref(total), dev.ptr(work), work.numel(), s),
-              "transpose_count")
+    dev.check(L.op2hip_transpose_count_places(nrows, dev.ptr(mv), m.arity, iter_size, dev.ptr(inc_ptr),
+                                              ctypes.byref(total), dev.ptr(places), dev.ptr(work),
+                                              work.numel(), s), "transpose_count")
     inc_ent = dev.empty((max(total.value, 1),), np.int32)
-    dev.check(L.op2hip_transpose_fill(nrows, dev.ptr(mv), m.arity, iter_size, dev.ptr(inc_ptr),
-                                      dev.ptr(inc_ent), dev.ptr(work), work.numel(), s),
-              "transpose_fill")
+    dev.check(L.op2hip_transpose_fill_places(nrows, dev.ptr(mv), m.arity, iter_size, dev.ptr(inc_ptr),
+                                             dev.ptr(places), dev.ptr(inc_ent), s), "transpose_fill")
     tr = Transpose(inc_ptr, inc_ent, int(total.value))
     m._cache[key] = tr
     return tr
