@@ -198,6 +198,31 @@ int op2hip_transpose_fill_places(int32_t nrows, const int32_t *map, int32_t arit
                                  int32_t iter_size, const int32_t *inc_ptr,
                                  const int32_t *places, int32_t *inc_ent, void *stream);
 
+/* ---- tiles of consecutive elements (generated loops) -------------------- */
+/* table: n x arity targets (device, none negative); tile b has the elements
+ * [b * tile, (b + 1) * tile), at most OP2HIP_TILE_CANDIDATES candidates.
+ * count: counts[b], the distinct targets of tile b.  fill: with tile_ptr the
+ * exclusive sums of the counts, nodes[tile_ptr[b] ..], tile b's targets
+ * ascending, and local (n x arity), every entry's place among them.
+ * add: out[r * dim + j] += the sum over r's slots (slots[ptr[r] .. ptr[r+1]),
+ * in that order) of partials[slot * dim + j], for outputs of type 0 float64,
+ * 1 float32 (both with float64 partials), 2 int32, 3 int64. */
+#define OP2HIP_TILE_CANDIDATES 4096
+int op2hip_tile_targets_count(int32_t n, int32_t tile, const int32_t *table, int32_t arity,
+                              int32_t *counts, void *stream);
+int op2hip_tile_targets_fill(int32_t n, int32_t tile, const int32_t *table, int32_t arity,
+                             const int32_t *tile_ptr, int32_t *nodes, uint16_t *local,
+                             void *stream);
+int op2hip_tile_targets_add(int32_t type, int32_t nrows, int32_t dim, const int32_t *ptr,
+                            const int32_t *slots, const void *partials, void *out,
+                            void *stream);
+/* slots[e][i][j]: position of block (rmap[e][i], cmap[e][j]) in the pattern;
+ * *bad counts the entries that are not in it (device int32, zeroed by the
+ * caller). */
+int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
+                     const int32_t *rmap, int32_t rarity, const int32_t *cmap, int32_t carity,
+                     int32_t *slots, int32_t *bad, void *stream);
+
 /* ---- sparsity (replaces pyop2/sparsity.pyx:121-284, build_sparsity and
  *      fill_with_zeros, non-extruded, one DataSet pair) ------------------ */
 /* Block pattern of the union over `pairs` of rmap[e,:] x cmap[e,:] for

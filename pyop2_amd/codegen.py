@@ -9,7 +9,7 @@ semantics (``pyop2/codegen/builder.py``):
   ``buf[i*dim + j] = dat[map[n][i]*dim + j]``; INC/WRITE buffers start at
   zero; direct Dats pass ``&dat[n*dim]``;
 * Globals: READ passes the device array; INC uses a zeroed buffer and
-  MIN/MAX a copy, reduced over the wavefront before one atomic per wave;
+  MIN/MAX a copy, reduced over the workgroup (``_REDUCE_BLOCKS``);
 * Mats: a zeroed ``(ar_r*rdim) x (ar_c*cdim)`` buffer, added (INC) or
   stored (WRITE) block by block at the slot found by binary search of the
   row's sorted column indices;
@@ -21,8 +21,11 @@ semantics (``pyop2/codegen/builder.py``):
 
 Indirect WRITE/RW arguments and Mat WRITE need exclusive targets, so such
 loops run coloured (greedy colouring, one launch per colour); INC-only
-loops run with atomics.  Sources are compiled for gfx950 with hiprtc and
-the code objects cached in memory and under ``<cache_dir>/hip``.
+loops run with atomics, or in tiles (``_Tiling``): a workgroup adds the
+increments of consecutive elements up in LDS, writes one partial sum per
+distinct target, and a second pass adds a target's partial sums.  Sources
+are compiled for gfx950 with hiprtc and the code objects cached in memory
+and under ``<cache_dir>/hip``.
 """
 import ctypes
 import hashlib
@@ -201,14 +204,18 @@ def _region_bounds(region, periodic=False):
     return "bottom_", "cend_"
 
 
-def generate_source(gk, map_index, block_flags=None):
+def generate_source(gk, map_index, block_flags=None, tiled=None):
     """HIP source of the wrapper kernel ``op2_wrap`` for GlobalKernel ``gk``.
 
     ``map_index[(arg, j)]`` is the position of an argument's j-th map in the
     unique-map list; ``block_flags[arg]`` says whether a Mat argument is
-    stored as BSR (else scalar CSR over dofs).
+    stored as BSR (else scalar CSR over dofs).  ``tiled`` (argument -> plan
+    number) makes the tiled form: the increments of those arguments go to
+    LDS accumulators through the plan's local ids and leave the workgroup as
+    partial sums.
     """
     block_flags = block_flags or {}
+    tiled = tiled or {}
     lk = gk.local_kernel
     extruded = getattr(gk, "_extruded", False)
     region = getattr(gk, "_iteration_region", None) if extruded else None
@@ -254,6 +261,8 @@ def generate_source(gk, map_index, block_flags=None):
     code = _strip_headers(lk.code)
     params = ["int32_t lo", "int32_t hi", "const int32_t *__restrict__ list", "int32_t atomic"]
     pre, call, post, red = [], [], [], []
+    accs = []            # (argument, plan, values per target) of the tiled form
+    reduced = []         # (argument, element type, components, operation) of the reduced Globals
     nmaps = len(set(map_index.values()))
     for k, (larg, garg) in enumerate(zip(lk.arguments, gk.arguments)):
         acc = larg.access
@@ -282,6 +291,12 @@ def generate_source(gk, map_index, block_flags=None):
             call.append(f"op2_ptr_{{(void *)buf{k}}}")
             if acc == READ:
                 continue
+            if k in tiled:
+                accs.append((k, tiled[k], dim))
+                post.append(f"    for (int i = 0; i < {ar}; ++i) {{ const int l_ = loc{tiled[k]}_[(int64_t)(n - base_) * {ar} + i];"
+                            f" for (int j = 0; j < {dim}; ++j) op2_atomic_add(&acc{k}_[l_ * {dim} + j],"
+                            f" ({_acc_type(t)})buf{k}[i * {dim} + j]); }}")
+                continue
             tgt = f"arg{k}[(int64_t)mi{k}[i] * {stride} + {comp} + j]"
             val = f"buf{k}[i * {dim} + j]"
             post.append(f"    for (int i = 0; i < {ear}; ++i) {{ if (mi{k}[i] < 0) continue;"
@@ -292,20 +307,21 @@ def generate_source(gk, map_index, block_flags=None):
             if acc == READ:
                 call.append(f"op2_ptr_{{(void *)arg{k}}}")
                 continue
-            # declared before the element guard so every lane takes part in the reduction
-            if acc == INC:
-                red.append(("decl", f"  {t} buf{k}[{dim}];\n  for (int q = 0; q < {dim}; ++q) buf{k}[q] = ({t})0;"))
-            else:
-                red.append(("decl", f"  {t} buf{k}[{dim}];\n  for (int q = 0; q < {dim}; ++q) buf{k}[q] = arg{k}[q];"))
+            # a buffer per element, as for the other outputs, added to the
+            # thread's result after it
+            start = f"({t})0" if acc == INC else f"arg{k}[q]"
+            join = {INC: "sum{k}_[q] + buf{k}[q]", MIN: "op2_min(sum{k}_[q], buf{k}[q])",
+                    MAX: "op2_max(sum{k}_[q], buf{k}[q])"}.get(acc, "").format(k=k)
+            red.append((f"  {t} sum{k}_[{dim}];\n  for (int q = 0; q < {dim}; ++q) sum{k}_[q] = {start};",
+                        f"    {t} buf{k}[{dim}];\n    for (int q = 0; q < {dim}; ++q) buf{k}[q] = {start};",
+                        f"    for (int q = 0; q < {dim}; ++q) sum{k}_[q] = {join};"))
             call.append(f"op2_ptr_{{(void *)buf{k}}}")
             fn = {INC: "sum", MIN: "min", MAX: "max"}.get(acc)
             if fn is None:
                 raise NotImplementedError(f"Global access {acc!r} in a par_loop")
             if t in _SHUFFLE_T:
                 raise NotImplementedError(f"Global reductions of {t} are not supported on the device")
-            aop = {INC: "op2_atomic_add", MIN: "op2_atomic_min", MAX: "op2_atomic_max"}[acc]
-            red.append(("post", f"  for (int q = 0; q < {dim}; ++q) {{ {t} v = op2_wave_{fn}(buf{k}[q]);"
-                                f" if (lane == 0) {aop}(&arg{k}[q], v); }}"))
+            reduced.append((k, t, dim, fn))
         elif isinstance(garg, MixedDatKernelArg):
             # one buffer: the packs of the components one after the other
             comps = garg.arguments
@@ -391,7 +407,16 @@ def generate_source(gk, map_index, block_flags=None):
                 store = "if (atomic) op2_atomic_add(&{tgt}, {val}); else {tgt} += {val};"
             else:
                 store = "{tgt} = {val};"
-            if block:
+            if k in tiled:
+                # targets are the blocks of the pattern, one local id per (i, j)
+                accs.append((k, tiled[k], rd * cd))
+                post.append(
+                    f"    for (int i = 0; i < {rar}; ++i) for (int j = 0; j < {car}; ++j) {{"
+                    f" const int l_ = loc{tiled[k]}_[(int64_t)(n - base_) * {rar * car} + i * {car} + j];"
+                    f" for (int ri = 0; ri < {rd}; ++ri) for (int cj = 0; cj < {cd}; ++cj)"
+                    f" op2_atomic_add(&acc{k}_[l_ * {rd * cd} + ri * {cd} + cj],"
+                    f" ({_acc_type(t)})buf{k}[(i * {rd} + ri) * {ncol} + j * {cd} + cj]); }}")
+            elif block:
                 tgt = f"arg{k}[(int64_t)s_ * {rd * cd} + ri * {cd} + cj]"
                 val = f"buf{k}[(i * {rd} + ri) * {ncol} + j * {cd} + cj]"
                 post.append(
@@ -418,8 +443,27 @@ def generate_source(gk, map_index, block_flags=None):
                for m, o in sorted(offsets.items())]
     offdecl += [f"    const int32_t quo{m}[{len(o)}] = {{{', '.join(str(int(v)) for v in o)}}};"
                 for m, o in sorted(quots.items())]
-    decls = "\n".join(s for kind, s in red if kind == "decl")
-    reds = "\n".join(s for kind, s in red if kind == "post")
+    params += [f"{t} *__restrict__ red{k}_" for k, t, _, _ in reduced]
+    if accs:
+        plans_used = sorted({g for _, g, _ in accs})
+        params += ["int32_t tile_", "int32_t base_"]
+        params += [p for g in plans_used for p in (f"const int32_t *__restrict__ tptr{g}_",
+                                                   f"const uint16_t *__restrict__ loc{g}_")]
+        params += [f"{_acc_type(_arg_ctype(lk, k))} *__restrict__ part{k}_" for k, _, _ in accs]
+        head = _tiled_head(lk, accs, plans_used)
+        loop = ["  for (int64_t t_ = first_ + threadIdx.x; t_ < last_; t_ += blockDim.x) {",
+                "    const int32_t n = (int32_t)t_;"]
+        tail = _tiled_tail(accs)
+    elif reduced:
+        # a workgroup runs several elements a lane, so that few partial
+        # results leave it
+        head, tail = [], []
+        loop = ["  for (int64_t t_ = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t_ < hi;"
+                " t_ += (int64_t)gridDim.x * blockDim.x) {",
+                "    const int32_t n = list ? list[t_] : (int32_t)t_;"]
+    else:
+        head, tail = ["  const int32_t t_ = lo + (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);"], []
+        loop = ["  if (t_ < hi) {", "    const int32_t n = list ? list[t_] : t_;"]
     src = [_PRELUDE,
            "#pragma clang force_cuda_host_device begin",
            headers, code,
@@ -427,13 +471,11 @@ def generate_source(gk, map_index, block_flags=None):
            'extern "C" __global__ void __launch_bounds__(256)',
            "op2_wrap(" + ", ".join(params) + ")",
            "{",
-           "  const int32_t t_ = lo + (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);",
-           "  const bool active = t_ < hi;",
-           "  const int lane = threadIdx.x & 63;",
-           "  (void)lane; (void)status;",
-           decls,
-           "  if (active) {",
-           "    const int32_t n = list ? list[t_] : t_;",
+           "  (void)status;",
+           *[d for d, _, _ in red],
+           *head,
+           *loop,
+           *[d for _, d, _ in red],
            *([] if not extruded else [
                *offdecl,
                "    const int32_t lay_ = %s;" % ("0" if gk._constant_layers else "n"),
@@ -448,10 +490,102 @@ def generate_source(gk, map_index, block_flags=None):
            f"    {lk.name}({', '.join(call + (['layer_'] if getattr(gk, '_pass_layer_arg', False) else []))});",
            *post,
            *(["    }"] if extruded else []),
+           *[d for _, _, d in red],
            "  }",
-           reds,
-           "}"]
+           *tail,
+           *_reduction_tail(reduced),
+           "}",
+           *_finish_kernel(reduced)]
     return "\n".join(s for s in src if s is not None)
+
+
+def _acc_type(t):
+    """Type the increments of a tile are added up in: float64 for floats
+    (LDS float32 adds run at a quarter of the float64 rate on gfx950)."""
+    return "double" if t in ("float", "double") else t
+
+
+def _arg_ctype(lk, k):
+    return as_cstr(np.dtype(lk.arguments[k].dtype))
+
+
+def _tiled_head(lk, accs, plans_used):
+    """The workgroup's tile, its accumulators in LDS, zeroed.  Each XCD takes
+    a contiguous range of tiles (workgroups go to the 8 XCDs in turn), so
+    that neighbouring tiles' shared targets meet in one L2."""
+    out = ["  extern __shared__ double smem_[];",
+           "  const int32_t q_ = (int32_t)gridDim.x / 8, m_ = (int32_t)gridDim.x % 8, x_ = (int32_t)blockIdx.x % 8;",
+           "  const int32_t b_ = x_ * q_ + (x_ < m_ ? x_ : m_) + (int32_t)blockIdx.x / 8;",
+           "  const int64_t first_ = lo + (int64_t)b_ * tile_;",
+           "  const int64_t last_ = first_ + tile_ < hi ? first_ + tile_ : hi;"]
+    out += [f"  const int32_t p{g}_ = tptr{g}_[b_], u{g}_ = tptr{g}_[b_ + 1] - p{g}_;" for g in plans_used]
+    out.append("  double *free_ = smem_;")
+    for k, g, dim in accs:
+        t = _acc_type(_arg_ctype(lk, k))
+        out += [f"  {t} *acc{k}_ = reinterpret_cast<{t} *>(free_);", f"  free_ += u{g}_ * {dim};",
+                f"  for (int32_t i = threadIdx.x; i < u{g}_ * {dim}; i += blockDim.x) acc{k}_[i] = ({t})0;"]
+    out.append("  __syncthreads();")
+    return out
+
+
+def _tiled_tail(accs):
+    """Every accumulator to its partial slot, contiguous per tile."""
+    out = ["  __syncthreads();"]
+    out += [f"  for (int32_t i = threadIdx.x; i < u{g}_ * {dim}; i += blockDim.x)"
+            f" part{k}_[(int64_t)p{g}_ * {dim} + i] = acc{k}_[i];" for k, g, dim in accs]
+    return out
+
+
+def _reduction_tail(reduced):
+    """Each reduced Global over the workgroup: waves, then LDS, then one
+    partial result (or, for launches of few workgroups, one atomic)."""
+    out = []
+    if reduced:
+        out.append("  const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6, waves_ = (blockDim.x + 63) >> 6;")
+    for k, t, dim, fn in reduced:
+        step = {"sum": "w + buf", "min": "op2_min(w, buf)", "max": "op2_max(w, buf)"}[fn].replace("buf", f"s{k}_[v]")
+        atomic = {"sum": "op2_atomic_add", "min": "op2_atomic_min", "max": "op2_atomic_max"}[fn]
+        out += [f"  __shared__ {t} s{k}_[4];",
+                f"  for (int q = 0; q < {dim}; ++q) {{",
+                f"    {t} w = op2_wave_{fn}(sum{k}_[q]);",
+                f"    if (lane_ == 0) s{k}_[wave_] = w;",
+                "    __syncthreads();",
+                "    if (threadIdx.x == 0) {",
+                f"      for (int v = 1; v < waves_; ++v) w = {step};",
+                f"      if (red{k}_) red{k}_[(int64_t)q * gridDim.x + blockIdx.x] = w; else {atomic}(&arg{k}[q], w);",
+                "    }",
+                "    __syncthreads();",
+                "  }"]
+    return out
+
+
+def _finish_kernel(reduced):
+    """``op2_finish``: one workgroup per component adds (or takes the minimum
+    or maximum of) the partial results of ``n`` workgroups."""
+    if not reduced:
+        return []
+    params = ", ".join(f"{t} *__restrict__ arg{k}, const {t} *__restrict__ red{k}_" for k, t, _, _ in reduced)
+    out = ['extern "C" __global__ void __launch_bounds__(256)', f"op2_finish(int32_t n, {params})", "{",
+           "  int c = blockIdx.x;", "  const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;"]
+    for k, t, dim, fn in reduced:
+        start = f"({t})0" if fn == "sum" else f"arg{k}[c]"
+        join = {"sum": "{a} + {b}", "min": "op2_min({a}, {b})", "max": "op2_max({a}, {b})"}[fn]
+        out += [f"  __shared__ {t} s{k}_[4];",
+                f"  if (c >= 0 && c < {dim}) {{",
+                f"    {t} w = {start};",
+                "    for (int32_t i = threadIdx.x; i < n; i += 256) w = "
+                + join.format(a="w", b=f"red{k}_[(int64_t)c * n + i]") + ";",
+                f"    w = op2_wave_{fn}(w);",
+                f"    if (lane_ == 0) s{k}_[wave_] = w;",
+                "    __syncthreads();",
+                "    if (threadIdx.x == 0) {",
+                "      for (int v = 1; v < 4; ++v) w = " + join.format(a="w", b=f"s{k}_[v]") + ";",
+                f"      arg{k}[c] = " + (join.format(a=f"arg{k}[c]", b="w")) + ";",
+                "    }",
+                "  }",
+                f"  c -= {dim};"]
+    out.append("}")
+    return out
 
 
 _gen_lock = threading.Lock()
@@ -506,6 +640,25 @@ def _module(src):
     return mod
 
 
+# Workgroups of a launch that reduces into Globals: each adds up its elements
+# and leaves one partial result per component, which op2_finish adds (one
+# atomic per wave on a Global's one address takes 52 ns after the other: 295 of
+# 310 us for 361,201 elements); up to _ATOMIC_BLOCKS workgroups send atomics,
+# cheaper than the second launch.
+_REDUCE_BLOCKS = 2048
+_ATOMIC_BLOCKS = 16
+
+# Least increments of a loop that runs in tiles: below, device atomics hide
+# behind the host's issue of the call, and the second pass costs one launch more
+# (a call of 1.4 and 2.9 million increments of a P1 matrix kernel takes 75 and
+# 118 us with atomics, 62 and 65 us in tiles; of 1.9 and 3.8 million increments
+# of an edge flux, 77 and 149 against 101 us).  Most distinct targets per
+# increment: with less reuse a partial sum costs as much as an atomic.
+_TILED_LEAST = 1 << 21
+_TILED_REUSE = 0.75
+_TILED_TYPES = frozenset(("float64", "float32", "int32", "int64"))
+
+
 class GeneratedKernel:
     """Executor of a generated wrapper (``(start, end, ptrs, parloop)``)."""
 
@@ -516,6 +669,40 @@ class GeneratedKernel:
         self.strategy_used = None
         self._src = {}
         self._mods = {}
+        lk = gk.local_kernel
+        # components of every reduced Global
+        self._reduced = [(k, int(np.prod(garg.dim)) if len(garg.dim) else 1)
+                         for k, (larg, garg) in enumerate(zip(lk.arguments, gk.arguments))
+                         if isinstance(garg, GlobalKernelArg) and larg.access != READ]
+        self._tile_dims = self._tileable()
+
+    def _tileable(self):
+        """Values per target of every argument whose increments a tile can
+        add up (``{arg: dim}``; None if the loop has another kind of indirect
+        output, or none)."""
+        gk, lk = self.gk, self.gk.local_kernel
+        if getattr(gk, "_extruded", False) or gk._subset:
+            return None
+        out = {}
+        for k, (larg, garg) in enumerate(zip(lk.arguments, gk.arguments)):
+            if isinstance(garg, (MixedDatKernelArg, MixedMatKernelArg)):
+                return None
+            if isinstance(garg, DatKernelArg):
+                if garg.map_ is None or larg.access == READ:
+                    continue
+                if larg.access != INC or garg.index is not None or garg.map_.offset is not None:
+                    return None
+                dim = int(np.prod(garg.dim))
+            elif isinstance(garg, MatKernelArg):
+                if larg.access != INC or garg.unroll or any(m.offset is not None for m in garg.maps):
+                    return None
+                dim = int(np.prod(garg.dims[0][0]))
+            else:
+                continue
+            if np.dtype(larg.dtype).name not in _TILED_TYPES:
+                return None
+            out[k] = dim
+        return out or None
 
     def _unique_maps(self, parloop):
         seen, index = [], {}
@@ -539,13 +726,52 @@ class GeneratedKernel:
                 out.append((k, tuple(getattr(b, "_gen_flag", b._block) for b in a.data)))
         return tuple(out)
 
-    def source(self, parloop):
+    def source(self, parloop, groups=()):
+        """The wrapper's source; ``groups``, the (argument, plan) pairs of
+        the tiled form."""
         flags = self._flags(parloop)
-        src = self._src.get(flags)
+        src = self._src.get((flags, groups))
         if src is None:
             _, index = self._unique_maps(parloop)
-            src = self._src[flags] = generate_source(self.gk, index, dict(flags))
+            src = self._src[flags, groups] = generate_source(self.gk, index, dict(flags), dict(groups))
         return src
+
+    def _loaded(self, parloop, flags, groups=()):
+        mod = self._mods.get((flags, groups))
+        if mod is None:
+            mod = self._mods[flags, groups] = _module(self.source(parloop, groups))
+        return mod
+
+    def _tiles(self, parloop, start, end):
+        """The loop's tiling (``plans.target_tiles``) and its (argument,
+        plan) pairs when it runs in tiles: large enough, every target
+        present, and targets shared by a tile's elements often enough; else
+        None and no pairs."""
+        if (self._tile_dims is None or configuration["strategy"] not in ("auto", "staged") or end <= start
+                or isinstance(parloop.iterset, Subset)):
+            return None, ()
+        from pyop2_amd import plans
+        targets, groups, width = [], [], 0
+        for k, dim in self._tile_dims.items():
+            a = parloop.arguments[k]
+            if any(m.has_negative for m in a.maps):
+                return None, ()
+            if a.kind == "mat":
+                if hasattr(a.data, "_gen_flag") or (dim > 1 and not a.data._block):
+                    return None, ()
+                target = (a.maps[0], a.maps[1], a.data)
+                width += a.maps[0].arity * a.maps[1].arity * dim
+            else:
+                target = (a.maps[0], None, None)
+                width += a.maps[0].arity * dim
+            g = next((i for i, t in enumerate(targets) if all(x is y for x, y in zip(t, target))), len(targets))
+            if g == len(targets):
+                targets.append(target)
+            groups.append((k, g))
+        if (end - start) * width < _TILED_LEAST:
+            return None, ()
+        tiles = plans.target_tiles(targets, start, end, width, _TILED_REUSE)
+        return tiles, tuple(groups) if tiles is not None else ()
 
     def _conflict_maps(self, parloop):
         """Maps whose targets must be exclusive within a launch."""
@@ -576,9 +802,8 @@ class GeneratedKernel:
         if parloop is None:
             raise RuntimeError("generated loops are launched by a Parloop")
         flags = self._flags(parloop)
-        mod = self._mods.get(flags)
-        if mod is None:
-            mod = self._mods[flags] = _module(self.source(parloop))
+        tiles, groups = self._tiles(parloop, start, end)
+        mod = self._loaded(parloop, flags, groups)
         maps, _ = self._unique_maps(parloop)
         conflict, need_colour = self._conflict_maps(parloop)
         if configuration["strategy"] == "coloured" and not need_colour:
@@ -620,16 +845,33 @@ class GeneratedKernel:
                 if getattr(m, "offset", None) is not None:
                     m.check_extruded(iterset, region)
             vals.append(ctypes.c_void_p(dev.ptr(iterset.device_layers)))
-        L = dev.lib()
+        L, lk = dev.lib(), self.gk.local_kernel
         s = dev.stream()
 
-        def launch(lo, hi, lst, atomic):
-            allv = [ctypes.c_int32(lo), ctypes.c_int32(hi), ctypes.c_void_p(lst), ctypes.c_int32(atomic)] + vals
+        def raw_launch(name, grid, block, lds, allv):
             argv = (ctypes.c_void_p * len(allv))(*[ctypes.addressof(v) for v in allv])
-            grid = (hi - lo + self.BLOCK - 1) // self.BLOCK
+            dev.check(L.op2hip_jit_launch(mod, name, grid, block, lds, argv, s),
+                      f"launch of generated {self.gk.name}")
+
+        def launch(lo, hi, lst, atomic, grid=None, block=self.BLOCK, lds=0, extra=()):
+            if grid is None:
+                grid = (hi - lo + self.BLOCK - 1) // self.BLOCK
+                if self._reduced:
+                    grid = min(grid, _REDUCE_BLOCKS)
+            head = [ctypes.c_int32(lo), ctypes.c_int32(hi), ctypes.c_void_p(lst), ctypes.c_int32(atomic)]
+            parts = []
+            if self._reduced:
+                # partial results of the workgroups, gone when the stream is done with them
+                parts = [dev.empty((dim * grid,), lk.arguments[k].dtype) if grid > _ATOMIC_BLOCKS else None
+                         for k, dim in self._reduced]
+            reds = [ctypes.c_void_p(dev.ptr(p)) for p in parts]
             with dev.timed_launch("op2_wrap:" + self.gk.name):
-                rc = L.op2hip_jit_launch(mod, b"op2_wrap", grid, self.BLOCK, 0, argv, s)
-            dev.check(rc, f"launch of generated {self.gk.name}")
+                raw_launch(b"op2_wrap", grid, block, lds, head + vals + reds + list(extra))
+                if self._reduced and grid > _ATOMIC_BLOCKS:
+                    pairs = [v for (k, _), r in zip(self._reduced, reds)
+                             for v in (ctypes.c_void_p(dev.ptr(parloop.arguments[k].data._device_array())), r)]
+                    raw_launch(b"op2_finish", sum(d for _, d in self._reduced), self.BLOCK, 0,
+                               [ctypes.c_int32(grid)] + pairs)
 
         if need_colour and conflict:
             from pyop2_amd import plans
@@ -656,10 +898,37 @@ class GeneratedKernel:
                 if hi > lo:
                     launch(lo, hi, ep, 0)
             self.strategy_used = "coloured"
+        elif tiles is not None:
+            self._launch_tiles(tiles, groups, start, end, parloop, launch)
+            self.strategy_used = "staged"
         else:
             lst = dev.ptr(iterset.device_indices) if isinstance(iterset, Subset) else 0
             launch(start, end, lst, 1)
             self.strategy_used = "atomic"
+
+    def _launch_tiles(self, tiles, groups, start, end, parloop, launch):
+        """The tiles' launch, then one pass per output that adds its targets'
+        partial sums (float64 for floats)."""
+        L, lk = dev.lib(), self.gk.local_kernel
+        plan_args = [ctypes.c_int32(tiles.tile), ctypes.c_int32(start)]
+        for p in tiles.plans:
+            plan_args += [ctypes.c_void_p(dev.ptr(p.tile_ptr)), ctypes.c_void_p(dev.ptr(p.local))]
+        parts, lds = [], 0
+        for k, g in groups:
+            dim, dt = self._tile_dims[k], np.dtype(lk.arguments[k].dtype)
+            acc = np.dtype(np.float64) if dt.kind == "f" else dt
+            parts.append((k, g, dim, dt, dev.empty((max(tiles.plans[g].nslots * dim, 1),), acc)))
+            lds += tiles.plans[g].max_targets * dim * 8
+        launch(start, end, 0, 1, tiles.ntiles, tiles.block, lds,
+               plan_args + [ctypes.c_void_p(dev.ptr(p[4])) for p in parts])
+        for k, g, dim, dt, part in parts:
+            p, data = tiles.plans[g], parloop.arguments[k].data
+            out = data.device_values if parloop.arguments[k].kind == "mat" else data._device_array()
+            with dev.timed_launch("op2_wrap:" + self.gk.name):
+                rc = L.op2hip_tile_targets_add({"float64": 0, "float32": 1, "int32": 2, "int64": 3}[dt.name],
+                                               p.nrows, dim, dev.ptr(p.row_ptr), dev.ptr(p.row_slots),
+                                               dev.ptr(part), dev.ptr(out), dev.stream())
+            dev.check(rc, f"partial sums of generated {self.gk.name}")
 
 
 class _ColumnTargets:

@@ -118,6 +118,10 @@ _SIGNATURES = {
     "op2hip_transpose_count_places": (ctypes.c_int, [_I, _V, _I, _I, _V, ctypes.POINTER(ctypes.c_int64),
                                                      _V, _V, ctypes.c_size_t, _V]),
     "op2hip_transpose_fill_places": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, _V]),
+    "op2hip_mat_slots": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _I, _V, _V, _V]),
+    "op2hip_tile_targets_count": (ctypes.c_int, [_I, _I, _V, _I, _V, _V]),
+    "op2hip_tile_targets_fill": (ctypes.c_int, [_I, _I, _V, _I, _V, _V, _V, _V]),
+    "op2hip_tile_targets_add": (ctypes.c_int, [_I, _I, _I, _V, _V, _V, _V, _V]),
     "op2hip_transpose_fill": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, ctypes.c_size_t, _V]),
     "op2hip_sparsity_count": (ctypes.c_int, [_I, _I, _V, _I, _V, _V, _I, _V,
                                              ctypes.POINTER(ctypes.c_int64), _V, ctypes.c_size_t, _V]),

@@ -454,6 +454,108 @@ def tile_plan(maps, start, end, tile_size, node_cap=0):
 
 
 @dataclass
+class TargetPlan:
+    """Distinct targets of every tile of consecutive elements (ascending, at
+    slots ``tile_ptr[b] .. tile_ptr[b + 1]``), the elements' local ids in
+    their tile, and per target the slots that name it."""
+    tile_ptr: object     # device int32, ntiles + 1
+    local: object        # device uint16, elements x arity
+    nslots: int
+    max_targets: int
+    nrows: int
+    row_ptr: object      # device int32, nrows + 1
+    row_slots: object    # device int32, nslots
+
+
+@dataclass
+class TargetTiles:
+    """A generated loop's tiling: one TargetPlan per distinct output map."""
+    tile: int
+    ntiles: int
+    block: int
+    plans: list
+
+
+# Candidates (elements x arity) of a tile the plan kernels take, and the float64
+# accumulators that fit a workgroup's 64 KB if no two elements share a target.
+_TARGET_CANDIDATES = 4096
+_TARGET_ACCUMULATORS = 8192
+
+
+def target_tiles(targets, start, end, width, most):
+    """Tiling of the elements [start, end) over ``targets``: per plan (row
+    map, None, None), or (row map, column map, Mat) for the blocks of a Mat's
+    pattern; ``width`` values incremented per element.  None when a tile of 64
+    elements does not fit, a target is missing from the pattern, or a plan has
+    more than ``most`` distinct targets per increment.  Built on the device
+    and cached on the first map."""
+    owner = targets[0][0]
+    key = ("targets", tuple((id(r), id(c), id(m.sparsity) if m is not None else 0, m._block if m is not None else 0)
+                            for r, c, m in targets), int(start), int(end), int(width))
+    hit = owner._cache.get(key)
+    if hit is not None:
+        return hit[0]
+    if dev.torch().cuda.is_current_stream_capturing():
+        return None   # a plan cannot be built (it reads sizes back) while a graph is captured
+    arities = [r.arity * (c.arity if c is not None else 1) for r, c, _ in targets]
+    tile = min(2048, min(_TARGET_CANDIDATES // a for a in arities), _TARGET_ACCUMULATORS // width) // 64 * 64
+    tiles = None
+    if tile:
+        made = []
+        for (r, c, m), arity in zip(targets, arities):
+            p = _target_plan(r, c, m, arity, start, end, tile, most)
+            if p is None:
+                break
+            made.append(p)
+        else:
+            tiles = TargetTiles(tile, -(-(end - start) // tile), min(256, tile), made)
+    # the maps and patterns of the key stay alive with it
+    owner._cache[key] = (tiles, [(r, c, m.sparsity if m is not None else None) for r, c, m in targets])
+    return tiles
+
+
+def _target_plan(rmap, cmap, mat, arity, start, end, tile, most):
+    L, s = dev.lib(), dev.stream()
+    n, ntiles = end - start, -(-(end - start) // tile)
+    if mat is None:
+        nrows, table = rmap.toset.total_size, rmap.device_values[start:end]
+    else:
+        nrows = int(mat._nnz) if mat._values is not None else int(mat.colidx.numel())
+        table, bad = dev.empty((n, arity), np.int32), dev.zeros((1,), np.int32)
+        dev.check(L.op2hip_mat_slots(n, dev.ptr(mat.rowptr), dev.ptr(mat.colidx),
+                                     dev.ptr(rmap.device_values[start:end]), rmap.arity,
+                                     dev.ptr(cmap.device_values[start:end]), cmap.arity, dev.ptr(table),
+                                     dev.ptr(bad), s), "mat_slots")
+        if int(bad.item()):
+            return None
+    if n * arity >= 2 ** 31:
+        return None
+    counts, tile_ptr = dev.empty((ntiles,), np.int32), dev.empty((ntiles + 1,), np.int32)
+    dev.check(L.op2hip_tile_targets_count(n, tile, dev.ptr(table), arity, dev.ptr(counts), s),
+              "tile_targets_count")
+    need, total = ctypes.c_size_t(), ctypes.c_int64()
+    dev.check(L.op2hip_scan_workspace(ntiles, ctypes.byref(need)), "scan_workspace")
+    work = dev.workspace(need.value)
+    dev.check(L.op2hip_exclusive_scan(ntiles, dev.ptr(counts), dev.ptr(tile_ptr), ctypes.byref(total),
+                                      dev.ptr(work), work.numel(), s), "tile_targets scan")
+    nslots = int(total.value)
+    if nslots > most * n * arity:
+        return None
+    nodes, local = dev.empty((max(nslots, 1),), np.int32), dev.empty((n, arity), np.uint16)
+    dev.check(L.op2hip_tile_targets_fill(n, tile, dev.ptr(table), arity, dev.ptr(tile_ptr), dev.ptr(nodes),
+                                         dev.ptr(local), s), "tile_targets_fill")
+    dev.check(L.op2hip_transpose_workspace(nrows, ctypes.byref(need)), "transpose_workspace")
+    work, places = dev.workspace(need.value), dev.empty((max(nslots, 1),), np.int32)
+    row_ptr, row_slots = dev.empty((nrows + 1,), np.int32), dev.empty((max(nslots, 1),), np.int32)
+    dev.check(L.op2hip_transpose_count_places(nrows, dev.ptr(nodes), 1, nslots, dev.ptr(row_ptr),
+                                              ctypes.byref(total), dev.ptr(places), dev.ptr(work),
+                                              work.numel(), s), "tile_targets transpose")
+    dev.check(L.op2hip_transpose_fill_places(nrows, dev.ptr(nodes), 1, nslots, dev.ptr(row_ptr),
+                                             dev.ptr(places), dev.ptr(row_slots), s), "tile_targets transpose")
+    return TargetPlan(tile_ptr, local, nslots, int(counts.max().item()), nrows, row_ptr, row_slots)
+
+
+@dataclass
 class RowList:
     """Batches of rows in element-local order (op2hip_plan_row_list)."""
     nbatches: int
