@@ -22,6 +22,7 @@ import numpy as np
 from pyop2_amd import device as dev
 from pyop2_amd.configuration import configuration
 from pyop2_amd.exceptions import DeviceError
+from pyop2_amd.types.data_carrier import _DEVICE, _HOST
 from pyop2_amd.types.mat import Mat
 
 __all__ = ["BatchedLaplace", "BatchMesh"]
@@ -118,6 +119,10 @@ class BatchedLaplace:
             max_nodes = max(max_nodes, tp.max_nodes[0])
             self._keep += [tr, rb, hit, tp]
             self.meshes.append((A, R, X, u))
+        # what a call visits: Dats whose host copy may be newer, Mats, outputs
+        self._inputs = [d for _, R, X, u in self.meshes for d in (X, u, R)]
+        self._mats = [A for A, _, _, _ in self.meshes]
+        self._outputs = [R for _, R, _, _ in self.meshes]
         raw = (BatchMesh * max(len(descs), 1))(*descs)
         host = np.frombuffer(bytes(raw), dtype=np.uint8)
         self._descs = dev.to_device(host)
@@ -187,17 +192,17 @@ class BatchedLaplace:
         """One step: every mesh's assembly and residual increment.  The batch
         holds the device storage of its Dats and Mats (host-side changes are
         copied there first, as a par_loop does)."""
-        for A, R, X, u in self.meshes:
-            X._device_array()
-            u._device_array()
-            R._device_array()
+        for d in self._inputs:
+            if d._where == _HOST:
+                d._device_array()
+        for A in self._mats:
             A.change_assembly_state(Mat.ADD_VALUES)
         if self._graph is not None:
             with dev.timed_launch("batched_p1_laplace"):
                 self._graph.replay()
         else:
             self._launch()
-        for A, R, _, _ in self.meshes:
+        for R in self._outputs:
             R.halo_valid = False
-            R._device_modified()
-            R.increment_dat_version()
+            R._where = _DEVICE
+            R._version += 1

@@ -29,6 +29,7 @@ and under ``<cache_dir>/hip``.
 """
 import ctypes
 import hashlib
+import operator
 import os
 import re
 import threading
@@ -650,13 +651,14 @@ _ATOMIC_BLOCKS = 16
 
 # Least increments of a loop that runs in tiles: below, device atomics hide
 # behind the host's issue of the call, and the second pass costs one launch more
-# (a call of 1.4 and 2.9 million increments of a P1 matrix kernel takes 75 and
-# 118 us with atomics, 62 and 65 us in tiles; of 1.9 and 3.8 million increments
-# of an edge flux, 77 and 149 against 101 us).  Most distinct targets per
-# increment: with less reuse a partial sum costs as much as an atomic.
-_TILED_LEAST = 1 << 21
+# (a pass with a P1 matrix kernel of 0.35, 0.72 and 2.9 million increments takes
+# 33, 44 and 107 us with atomics, 32, 32 and 42 us in tiles; one with an edge
+# flux of 0.47, 0.96 and 3.8 million, 39, 44 and 149 against 46 us).  Most
+# distinct targets per increment: with less reuse a partial sum costs as much
+# as an atomic.
+_TILED_LEAST = 3 << 18
 _TILED_REUSE = 0.75
-_TILED_TYPES = frozenset(("float64", "float32", "int32", "int64"))
+_TILED_CODES = {"float64": 0, "float32": 1, "int32": 2, "int64": 3}
 
 
 class GeneratedKernel:
@@ -699,7 +701,7 @@ class GeneratedKernel:
                 dim = int(np.prod(garg.dims[0][0]))
             else:
                 continue
-            if np.dtype(larg.dtype).name not in _TILED_TYPES:
+            if np.dtype(larg.dtype).name not in _TILED_CODES:
                 return None
             out[k] = dim
         return out or None
@@ -801,13 +803,21 @@ class GeneratedKernel:
     def __call__(self, start, end, ptrs, parloop):
         if parloop is None:
             raise RuntimeError("generated loops are launched by a Parloop")
-        flags = self._flags(parloop)
-        tiles, groups = self._tiles(parloop, start, end)
-        mod = self._loaded(parloop, flags, groups)
-        maps, _ = self._unique_maps(parloop)
+        own = parloop.__dict__.setdefault("_launches", {})
+        launch = own.get((start, end, self))
+        if launch is None or not launch.holds(parloop):
+            launch = _GeneratedLaunch(self, start, end, parloop)
+            # tiles cannot be planned while a graph is captured: later calls may
+            if not dev.torch().cuda.is_current_stream_capturing():
+                own[(start, end, self)] = launch
+        launch(parloop)
+        self.strategy_used = launch.strategy
+
+    def _colours(self, start, end, parloop):
+        """The colour plan of a loop that runs coloured, else None."""
         conflict, need_colour = self._conflict_maps(parloop)
         if configuration["strategy"] == "coloured" and not need_colour:
-            conflict, _ = [], False
+            conflict = []
             for larg, garg, a in zip(self.gk.local_kernel.arguments, self.gk.arguments, parloop.arguments):
                 if (isinstance(garg, DatKernelArg) and garg.map_ is not None and larg.access != READ) \
                         or isinstance(garg, MatKernelArg):
@@ -817,118 +827,195 @@ class GeneratedKernel:
                 elif isinstance(garg, MixedMatKernelArg):
                     conflict.extend(a.maps[:garg.shape[0]])
             need_colour = bool(conflict)
-        vals = []
-        mat_status = []
-        for garg, a in zip(self.gk.arguments, parloop.arguments):
-            if isinstance(garg, MatKernelArg):
-                mat = a.data
-                vals += [ctypes.c_void_p(dev.ptr(mat.rowptr)), ctypes.c_void_p(dev.ptr(mat.colidx)),
-                         ctypes.c_void_p(dev.ptr(mat.device_values))]
-                mat_status.append(mat._status)
-            elif isinstance(garg, MixedMatKernelArg):
-                for blk in a.data:
-                    vals += [ctypes.c_void_p(dev.ptr(blk.rowptr)), ctypes.c_void_p(dev.ptr(blk.colidx)),
-                             ctypes.c_void_p(dev.ptr(blk.device_values))]
-                mat_status.append(a.data[0, 0]._status)
-            elif isinstance(garg, MixedDatKernelArg):
-                vals += [ctypes.c_void_p(dev.ptr(d._device_array())) for d in a.data]
-            else:
-                vals.append(ctypes.c_void_p(dev.ptr(a.data._device_array())))
-        vals += [ctypes.c_void_p(dev.ptr(m.device_values)) for m in maps]
-        status = mat_status[0] if mat_status else _dummy_status()
-        vals.append(ctypes.c_void_p(dev.ptr(status)))
+        if not (need_colour and conflict):
+            return None
+        from pyop2_amd import plans
+        iterset, region = parloop.iterset, getattr(self.gk, "_iteration_region", None)
+        if isinstance(iterset, Subset):
+            elems = iterset.indices[start:end]
+        else:
+            elems = np.arange(start, end, dtype=np.int32)
+        key = (iterset._plan_key(), start, end, tuple(id(m) for m in conflict), int(region or 0))
+        if not getattr(self.gk, "_extruded", False):
+            return plans.colour_plan(conflict[0], elems, [(m, id(m.toset)) for m in conflict], key)
+        # a column's targets over all its layers (a thread runs the
+        # layers of its column one after the other)
+        cols = np.ascontiguousarray(elems, dtype=np.int32)   # column ids, in launch order
+        targets = [(_ColumnTargets(m, iterset, cols, region), id(m.toset)) for m in conflict]
+        plan = plans.colour_plan(conflict[0], np.arange(len(cols), dtype=np.int32), targets,
+                                 ("extruded",) + key)
+        return _column_plan(plan, cols, conflict[0], ("extruded-cols",) + key)
+
+
+class _GeneratedLaunch:
+    """One band of a generated loop, ready but for the addresses of its data:
+    the loaded kernel, its argument block, and the colours or tiles it runs
+    by.  Held by the loop it was made for; ``holds`` says whether what it was
+    made from is still the loop's."""
+
+    def __init__(self, kernel, start, end, parloop):
+        self.kernel, self.start, self.end = kernel, start, end
+        gk = kernel.gk
+        self.lock = threading.Lock()
+        flags = kernel._flags(parloop)
+        tiles, self.groups = kernel._tiles(parloop, start, end)
+        self.tiles = tiles
+        self.mod = kernel._loaded(parloop, flags, self.groups)
+        maps, _ = kernel._unique_maps(parloop)
         iterset = parloop.iterset
-        extruded = getattr(self.gk, "_extruded", False)
-        if extruded:
-            region = getattr(self.gk, "_iteration_region", None)
+        self.made_for = self._made_of(parloop)
+        self.flags, self.strategies = flags, (configuration["strategy"], _TILED_LEAST)
+        # data arguments: (argument block entries, argument, what)
+        self.data, vals, self.status_of = [], [], None
+        for k, (garg, a) in enumerate(zip(gk.arguments, parloop.arguments)):
+            n = {True: 3, False: 1}[isinstance(garg, MatKernelArg)]
+            if isinstance(garg, MixedMatKernelArg):
+                n = 3 * sum(1 for _ in a.data)
+            elif isinstance(garg, MixedDatKernelArg):
+                n = sum(1 for _ in a.data)
+            if isinstance(garg, (MatKernelArg, MixedMatKernelArg)) and self.status_of is None:
+                self.status_of = k
+            slots = [ctypes.c_void_p() for _ in range(n)]
+            self.data.append((slots, k, garg))
+            vals += slots
+        vals += [ctypes.c_void_p(dev.ptr(m.device_values)) for m in maps]
+        self.keep = [m.device_values for m in maps]
+        self.status = ctypes.c_void_p(dev.ptr(_dummy_status()) if self.status_of is None else 0)
+        vals.append(self.status)
+        if getattr(gk, "_extruded", False):
+            region = getattr(gk, "_iteration_region", None)
             for m in maps:
                 if getattr(m, "offset", None) is not None:
                     m.check_extruded(iterset, region)
             vals.append(ctypes.c_void_p(dev.ptr(iterset.device_layers)))
-        L, lk = dev.lib(), self.gk.local_kernel
-        s = dev.stream()
+            self.keep.append(iterset.device_layers)
+        self.colours = kernel._colours(start, end, parloop)
+        self.list = 0
+        if isinstance(iterset, Subset):
+            self.list = dev.ptr(iterset.device_indices)
+            self.keep.append(iterset.device_indices)
+        self.strategy = "coloured" if self.colours else "staged" if tiles is not None else "atomic"
+        # the argument block: bounds, list, atomic flag, data, maps, partial
+        # results of the reduced Globals, and the tiles' plan and partial sums
+        self.head = [ctypes.c_int32(), ctypes.c_int32(), ctypes.c_void_p(), ctypes.c_int32()]
+        self.reds = [ctypes.c_void_p() for _ in kernel._reduced]
+        self.parts, extra, self.lds = [], [], 0
+        if tiles is not None:
+            extra = [ctypes.c_int32(tiles.tile), ctypes.c_int32(start)]
+            for p in tiles.plans:
+                extra += [ctypes.c_void_p(dev.ptr(p.tile_ptr)), ctypes.c_void_p(dev.ptr(p.local))]
+            for k, g in self.groups:
+                dt = np.dtype(gk.local_kernel.arguments[k].dtype)
+                plan, dim, slot = tiles.plans[g], kernel._tile_dims[k], ctypes.c_void_p()
+                acc = np.dtype(np.float64) if dt.kind == "f" else dt
+                self.parts.append((slot, k, plan, dim, _TILED_CODES[dt.name], acc))
+                self.lds += plan.max_targets * dim * 8
+                extra.append(slot)
+        block = self.head + vals + self.reds + extra
+        self.argv = (ctypes.c_void_p * len(block))(*[ctypes.addressof(v) for v in block])
+        self.block = block
+        self.count = ctypes.c_int32()
+        self.globals = [ctypes.c_void_p() for _ in kernel._reduced]
+        finish = [self.count] + [v for pair in zip(self.globals, self.reds) for v in pair]
+        self.finish = (ctypes.c_void_p * len(finish))(*[ctypes.addressof(v) for v in finish])
+        self.name = "op2_wrap:" + gk.name
 
-        def raw_launch(name, grid, block, lds, allv):
-            argv = (ctypes.c_void_p * len(allv))(*[ctypes.addressof(v) for v in allv])
-            dev.check(L.op2hip_jit_launch(mod, name, grid, block, lds, argv, s),
-                      f"launch of generated {self.gk.name}")
+    @staticmethod
+    def _made_of(parloop):
+        """Maps and patterns the launch's plans follow from."""
+        out = [parloop.iterset]
+        for a in parloop.arguments:
+            out += a.maps
+            if a.kind in ("mat", "mixed_mat"):
+                out.append(a.data.sparsity)
+        return out
 
-        def launch(lo, hi, lst, atomic, grid=None, block=self.BLOCK, lds=0, extra=()):
-            if grid is None:
-                grid = (hi - lo + self.BLOCK - 1) // self.BLOCK
-                if self._reduced:
-                    grid = min(grid, _REDUCE_BLOCKS)
-            head = [ctypes.c_int32(lo), ctypes.c_int32(hi), ctypes.c_void_p(lst), ctypes.c_int32(atomic)]
-            parts = []
-            if self._reduced:
-                # partial results of the workgroups, gone when the stream is done with them
-                parts = [dev.empty((dim * grid,), lk.arguments[k].dtype) if grid > _ATOMIC_BLOCKS else None
-                         for k, dim in self._reduced]
-            reds = [ctypes.c_void_p(dev.ptr(p)) for p in parts]
-            with dev.timed_launch("op2_wrap:" + self.gk.name):
-                raw_launch(b"op2_wrap", grid, block, lds, head + vals + reds + list(extra))
-                if self._reduced and grid > _ATOMIC_BLOCKS:
-                    pairs = [v for (k, _), r in zip(self._reduced, reds)
-                             for v in (ctypes.c_void_p(dev.ptr(parloop.arguments[k].data._device_array())), r)]
-                    raw_launch(b"op2_finish", sum(d for _, d in self._reduced), self.BLOCK, 0,
-                               [ctypes.c_int32(grid)] + pairs)
+    def holds(self, parloop):
+        now = self._made_of(parloop)
+        return (self.strategies == (configuration["strategy"], _TILED_LEAST) and len(now) == len(self.made_for)
+                and all(map(operator.is_, self.made_for, now))
+                and (self.status_of is None or self.flags == self.kernel._flags(parloop)))
 
-        if need_colour and conflict:
-            from pyop2_amd import plans
-            if isinstance(iterset, Subset):
-                elems = iterset.indices[start:end]
+    def _fill(self, parloop):
+        args = parloop.arguments
+        for slots, k, garg in self.data:
+            data = args[k].data
+            if isinstance(garg, MatKernelArg):
+                blocks = (data,)
+            elif isinstance(garg, MixedMatKernelArg):
+                blocks = tuple(data)
+            elif isinstance(garg, MixedDatKernelArg):
+                for s, d in zip(slots, data):
+                    s.value = d._device_array().data_ptr()
+                continue
             else:
-                elems = np.arange(start, end, dtype=np.int32)
-            key = (iterset._plan_key(), start, end, tuple(id(m) for m in conflict),
-                   int(getattr(self.gk, "_iteration_region", None) or 0))
-            if extruded:
-                # a column's targets over all its layers (a thread runs the
-                # layers of its column one after the other)
-                region = getattr(self.gk, "_iteration_region", None)
-                cols = np.ascontiguousarray(elems, dtype=np.int32)   # column ids, in launch order
-                targets = [(_ColumnTargets(m, iterset, cols, region), id(m.toset)) for m in conflict]
-                plan = plans.colour_plan(conflict[0], np.arange(len(cols), dtype=np.int32), targets,
-                                         ("extruded",) + key)
-                plan = _column_plan(plan, cols, conflict[0], ("extruded-cols",) + key)
-            else:
-                plan = plans.colour_plan(conflict[0], elems, [(m, id(m.toset)) for m in conflict], key)
-            ep = dev.ptr(plan.elems)
-            for c in range(plan.ncolours):
-                lo, hi = int(plan.offsets[c]), int(plan.offsets[c + 1])
-                if hi > lo:
-                    launch(lo, hi, ep, 0)
-            self.strategy_used = "coloured"
-        elif tiles is not None:
-            self._launch_tiles(tiles, groups, start, end, parloop, launch)
-            self.strategy_used = "staged"
-        else:
-            lst = dev.ptr(iterset.device_indices) if isinstance(iterset, Subset) else 0
-            launch(start, end, lst, 1)
-            self.strategy_used = "atomic"
+                slots[0].value = data._device_array().data_ptr()
+                continue
+            for i, b in enumerate(blocks):
+                slots[3 * i].value = b.rowptr.data_ptr()
+                slots[3 * i + 1].value = b.colidx.data_ptr()
+                slots[3 * i + 2].value = b.device_values.data_ptr()
+        if self.status_of is not None:
+            data = args[self.status_of].data
+            if isinstance(self.kernel.gk.arguments[self.status_of], MixedMatKernelArg):
+                data = data[0, 0]
+            self.status.value = data._status.data_ptr()
 
-    def _launch_tiles(self, tiles, groups, start, end, parloop, launch):
+    def __call__(self, parloop):
+        with self.lock:   # the argument block is this launch's own
+            self._fill(parloop)
+            with dev.timed_launch(self.name):
+                if self.colours is not None:
+                    plan = self.colours
+                    ep = dev.ptr(plan.elems)
+                    for c in range(plan.ncolours):
+                        lo, hi = int(plan.offsets[c]), int(plan.offsets[c + 1])
+                        if hi > lo:
+                            self._launch(parloop, lo, hi, ep, 0)
+                elif self.tiles is not None:
+                    self._launch_tiles(parloop)
+                else:
+                    self._launch(parloop, self.start, self.end, self.list, 1)
+
+    def _launch(self, parloop, lo, hi, lst, atomic, grid=0, block=GeneratedKernel.BLOCK, lds=0):
+        L, kernel, stream = dev.lib(), self.kernel, dev.raw_stream()
+        if not grid:
+            grid = (hi - lo + block - 1) // block
+            if self.reds:
+                grid = min(grid, _REDUCE_BLOCKS)
+        self.head[0].value, self.head[1].value, self.head[2].value, self.head[3].value = lo, hi, lst, atomic
+        finish = self.reds and grid > _ATOMIC_BLOCKS
+        if self.reds:
+            # partial results of the workgroups, free again behind the launches
+            parts = [dev.empty((dim * grid,), kernel.gk.local_kernel.arguments[k].dtype) if finish else None
+                     for k, dim in kernel._reduced]
+            for slot, p in zip(self.reds, parts):
+                slot.value = dev.ptr(p)
+        rc = L.op2hip_jit_launch(self.mod, b"op2_wrap", grid, block, lds, self.argv, stream)
+        if not rc and finish:
+            self.count.value = grid
+            for slot, (k, _) in zip(self.globals, kernel._reduced):
+                slot.value = parloop.arguments[k].data._device_array().data_ptr()
+            rc = L.op2hip_jit_launch(self.mod, b"op2_finish", sum(d for _, d in kernel._reduced),
+                                     GeneratedKernel.BLOCK, 0, self.finish, stream)
+        if rc:
+            dev.check(rc, f"launch of generated {kernel.gk.name}")
+
+    def _launch_tiles(self, parloop):
         """The tiles' launch, then one pass per output that adds its targets'
         partial sums (float64 for floats)."""
-        L, lk = dev.lib(), self.gk.local_kernel
-        plan_args = [ctypes.c_int32(tiles.tile), ctypes.c_int32(start)]
-        for p in tiles.plans:
-            plan_args += [ctypes.c_void_p(dev.ptr(p.tile_ptr)), ctypes.c_void_p(dev.ptr(p.local))]
-        parts, lds = [], 0
-        for k, g in groups:
-            dim, dt = self._tile_dims[k], np.dtype(lk.arguments[k].dtype)
-            acc = np.dtype(np.float64) if dt.kind == "f" else dt
-            parts.append((k, g, dim, dt, dev.empty((max(tiles.plans[g].nslots * dim, 1),), acc)))
-            lds += tiles.plans[g].max_targets * dim * 8
-        launch(start, end, 0, 1, tiles.ntiles, tiles.block, lds,
-               plan_args + [ctypes.c_void_p(dev.ptr(p[4])) for p in parts])
-        for k, g, dim, dt, part in parts:
-            p, data = tiles.plans[g], parloop.arguments[k].data
-            out = data.device_values if parloop.arguments[k].kind == "mat" else data._device_array()
-            with dev.timed_launch("op2_wrap:" + self.gk.name):
-                rc = L.op2hip_tile_targets_add({"float64": 0, "float32": 1, "int32": 2, "int64": 3}[dt.name],
-                                               p.nrows, dim, dev.ptr(p.row_ptr), dev.ptr(p.row_slots),
-                                               dev.ptr(part), dev.ptr(out), dev.stream())
-            dev.check(rc, f"partial sums of generated {self.gk.name}")
+        L, tiles = dev.lib(), self.tiles
+        bufs = [dev.empty((max(p.nslots * dim, 1),), acc) for _, _, p, dim, _, acc in self.parts]
+        for buf, part in zip(bufs, self.parts):
+            part[0].value = buf.data_ptr()
+        self._launch(parloop, self.start, self.end, 0, 1, tiles.ntiles, tiles.block, self.lds)
+        for buf, (_, k, p, dim, code, _) in zip(bufs, self.parts):
+            a = parloop.arguments[k]
+            out = a.data.device_values if a.kind == "mat" else a.data._device_array()
+            rc = L.op2hip_tile_targets_add(code, p.nrows, dim, dev.ptr(p.row_ptr), dev.ptr(p.row_slots),
+                                           buf.data_ptr(), out.data_ptr(), dev.raw_stream())
+            if rc:
+                dev.check(rc, f"partial sums of generated {self.kernel.gk.name}")
 
 
 class _ColumnTargets:

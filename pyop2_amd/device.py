@@ -11,6 +11,7 @@ import threading
 
 import numpy as np
 
+from pyop2_amd.configuration import configuration
 from pyop2_amd.exceptions import DeviceError, PatternError
 
 __all__ = ["lib", "torch", "device", "stream", "check", "ExecPlan", "MatDesc",
@@ -233,7 +234,6 @@ def available():
 def device():
     """The torch device all op2 data lives on (initialises it once)."""
     global _device_ready
-    from pyop2_amd.configuration import configuration
     t = torch()
     idx = configuration["device"]
     if not _device_ready:
@@ -247,10 +247,16 @@ def device():
     return t.device("cuda", idx)
 
 
+def raw_stream():
+    """Address of the current torch stream of the op2 device."""
+    if not _device_ready:
+        device()
+    return _torch._C._cuda_getCurrentRawStream(configuration["device"])
+
+
 def stream():
     """Current torch stream of the op2 device, as a void* for the C ABI."""
-    t = torch()
-    return ctypes.c_void_p(t.cuda.current_stream(device()).cuda_stream)
+    return ctypes.c_void_p(raw_stream())
 
 
 def check(rc, what=""):
@@ -362,6 +368,11 @@ class launch_timer:
     def __exit__(self, *exc):
         _timer.active = None
         return False
+
+
+def launch_timed():
+    """True while a launch_timer is active."""
+    return _timer.active is not None
 
 
 class timed_launch:

@@ -169,15 +169,10 @@ class GlobalKernel:
         if any(isinstance(garg, Constant) and larg.access is not READ
                for larg, garg in zip(local_kernel.arguments, arguments)):
             raise ValueError("Constants can only ever be read in a parloop, not modified")
-        counter = itertools.count()
-        seen_maps = collections.defaultdict(lambda: next(counter))
-        self.cache_key = (
-            local_kernel.cache_key,
-            *[a.cache_key for a in arguments],
-            *[seen_maps[m] for a in arguments for m in a.maps],
-            extruded, extruded_periodic, constant_layers, subset,
-            iteration_region, pass_layer_arg, configuration["simd_width"],
-        )
+        self.cache_key = self.key_of(local_kernel, arguments, extruded=extruded,
+                                     extruded_periodic=extruded_periodic, constant_layers=constant_layers,
+                                     subset=subset, iteration_region=iteration_region,
+                                     pass_layer_arg=pass_layer_arg)
         self.local_kernel = local_kernel
         self.arguments = arguments
         self._subset = subset
@@ -189,6 +184,19 @@ class GlobalKernel:
         self._iteration_region = iteration_region if extruded else None
         self._extruded_periodic = bool(extruded_periodic) and bool(extruded)
         self._executor = None
+
+    @staticmethod
+    def key_of(local_kernel, arguments, *, extruded=False, extruded_periodic=False, constant_layers=False,
+               subset=False, iteration_region=None, pass_layer_arg=False):
+        """Cache key of the GlobalKernel these arguments make."""
+        order = {}   # maps numbered in first-use order
+        return (
+            local_kernel.cache_key,
+            *[a.cache_key for a in arguments],
+            *[order.setdefault(m, len(order)) for a in arguments for m in a.maps],
+            extruded, extruded_periodic, constant_layers, subset,
+            iteration_region, pass_layer_arg, configuration["simd_width"],
+        )
 
     def __call__(self, comm, *args, parloop=None):
         """Execute over ``args = (start, end, *ptrs)`` on the current stream."""

@@ -236,7 +236,8 @@ class Parloop:
     def _static_parts(self):
         """What every call reads but only the bound arguments fix: the written
         arguments, the indirect Dats each exchange half visits (first use
-        order, each once), and whether any of them has a halo at all."""
+        order, each once), whether any of them has a halo at all, and the
+        objects that take a new version, a Mat state and a device mark."""
         st = self.__dict__.get("_static")
         if st is None:
             written = [(garg, arg, larg.access) for larg, garg, arg in self._triples()
@@ -246,29 +247,42 @@ class Parloop:
                 if isinstance(garg, (DatKernelArg, MixedDatKernelArg)) and garg.is_indirect:
                     exch.append((larg.access, arg.data))
             halo = any(data._has_halo() for _, data in exch)
-            st = self._static = (written, exch, halo)
+            versioned = [self.reduced_globals.get(arg.data, arg).data for _, arg, _ in written]
+            mats = [(arg.data, _INSERT_STATE[access]) for _, arg, access in written
+                    if arg.kind in ("mat", "mixed_mat")]
+            st = self._static = (written, exch, halo, versioned, mats)
         return st
 
     # -- running --------------------------------------------------------------------
     def _compute(self, part):
         """One band ``[part.offset, part.offset + part.size)``."""
         if part.size:
-            self.global_kernel(self.comm, part.offset, part.offset + part.size, *self.arglist,
-                               parloop=self)
+            gk = self.global_kernel
+            if type(gk) is GlobalKernel:
+                # its executors take the loop's data and maps from the loop
+                gk.compile()(part.offset, part.offset + part.size, (), self)
+            else:
+                gk(self.comm, part.offset, part.offset + part.size, *self.arglist, parloop=self)
 
     def compute(self):
         self()
 
     def __call__(self):
         self._prepare_outputs()
-        self._exchange("global_to_local_begin", _EXCHANGED_BEFORE)
-        self._compute(self.iterset.core_part)
-        self._exchange("global_to_local_end", _EXCHANGED_BEFORE)
-        self._compute(self.iterset.owned_part)
-        self._exchange("local_to_global_begin", _EXCHANGED_AFTER)
-        self._mark_outputs()
-        self._add_reductions()
-        self._exchange("local_to_global_end", _EXCHANGED_AFTER)
+        if self._static_parts()[2]:
+            self._exchange("global_to_local_begin", _EXCHANGED_BEFORE)
+            self._compute(self.iterset.core_part)
+            self._exchange("global_to_local_end", _EXCHANGED_BEFORE)
+            self._compute(self.iterset.owned_part)
+            self._exchange("local_to_global_begin", _EXCHANGED_AFTER)
+            self._mark_outputs()
+            self._add_reductions()
+            self._exchange("local_to_global_end", _EXCHANGED_AFTER)
+        else:   # no halo (one rank): nothing to exchange
+            self._compute(self.iterset.core_part)
+            self._compute(self.iterset.owned_part)
+            self._mark_outputs()
+            self._add_reductions()
 
     def _written(self):
         return self._static_parts()[0]
@@ -276,21 +290,20 @@ class Parloop:
     def _prepare_outputs(self):
         """New versions for written data (a temporary's Global is the one
         written), zeroed reduction temporaries, Mat insertion states."""
-        for garg, arg, access in self._written():
-            target = self.reduced_globals.get(arg.data, arg).data
+        _, _, _, versioned, mats = self._static_parts()
+        for target in versioned:
             target.increment_dat_version()
         for tmp in self.reduced_globals:
             tmp._device_array().zero_()
             tmp._device_modified()
-        for garg, arg, access in self._written():
-            if arg.kind in ("mat", "mixed_mat"):
-                arg.data.change_assembly_state(_INSERT_STATE[access])
+        for mat, state in mats:
+            mat.change_assembly_state(state)
 
     def _exchange(self, step, modes):
         """Calls ``step`` (a halo exchange half) once per distinct indirect Dat
         argument accessed with one of ``modes`` (nothing to do when none of
         them has a halo, as on one rank)."""
-        _, exch, halo = self._static_parts()
+        _, exch, halo = self._static_parts()[:3]
         if not halo:
             return
         done = []
@@ -452,11 +465,14 @@ _GLOBAL_KERNELS = {}
 def _shared_global_kernel(local_knl, kernel_args, **kwargs):
     """One GlobalKernel (and so one compiled executor) per cache key, as the
     reference reuses its compiled wrappers (``pyop2/compilation.py:427-489``)."""
-    gk = GlobalKernel(local_knl, kernel_args, **kwargs)
     try:
-        return _GLOBAL_KERNELS.setdefault(gk.cache_key, gk)
+        gk = _GLOBAL_KERNELS.get(GlobalKernel.key_of(local_knl, kernel_args, **kwargs))
     except TypeError:   # a key part that cannot be hashed: not shared
-        return gk
+        return GlobalKernel(local_knl, kernel_args, **kwargs)
+    if gk is None:
+        gk = GlobalKernel(local_knl, kernel_args, **kwargs)
+        gk = _GLOBAL_KERNELS.setdefault(gk.cache_key, gk)
+    return gk
 
 
 def LegacyParloop(local_knl, iterset, *args, **kwargs):

@@ -59,14 +59,15 @@ class validate_base:
         self._checks = checks
 
     def __call__(self, f):
+        code = inspect.unwrap(f).__code__   # stacked validators: the real signature
+        self.nargs = code.co_argcount
+        self.defaults = inspect.unwrap(f).__defaults__ or ()
+        self.varnames = code.co_varnames
+        self.file = code.co_filename
+        self.line = code.co_firstlineno + 1
+
         def wrapper(f, *args, **kwargs):
             if self._configuration_type_check():
-                code_of = inspect.unwrap(f)   # stacked validators: the real signature
-                self.nargs = code_of.__code__.co_argcount
-                self.defaults = code_of.__defaults__ or ()
-                self.varnames = code_of.__code__.co_varnames
-                self.file = code_of.__code__.co_filename
-                self.line = code_of.__code__.co_firstlineno + 1
                 self.check_args(args, kwargs)
             return f(*args, **kwargs)
         return _decorate(f, wrapper)
