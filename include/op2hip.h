@@ -57,12 +57,18 @@ enum op2hip_strategy {
                                   LDS once per batch, each output block
                                   evaluated and summed by one thread
                                   (op2hip_plan_cell_gather; no atomics) */
-  OP2HIP_ROWGATHER_ROWLIST = 8 /* as ROWGATHER_SLOTS over batches of rows taken
+  OP2HIP_ROWGATHER_ROWLIST = 8, /* as ROWGATHER_SLOTS over batches of rows taken
                                   in an element-local order instead of row-id
                                   order (op2hip_plan_row_list): the gathers of
                                   a batch stay in cache when the row numbering
                                   is scattered */
+  OP2HIP_ROWGATHER_TASKS = 9   /* row batches; each element's geometry staged in
+                                  LDS once per batch, element blocks summed in
+                                  registers over tasks of at most
+                                  OP2HIP_TASK_LENGTH blocks of one output block
+                                  (op2hip_task_plan_*); P2 elasticity matrix */
 };
+#define OP2HIP_TASK_LENGTH 6
 
 /* Execution plan of one launch.  Host struct; arrays as annotated. */
 typedef struct op2hip_exec {
@@ -132,6 +138,12 @@ typedef struct op2hip_exec {
      0-31 the incidence (element * 3 + i), 32-47 the row's block offset in
      the batch, 48-62 the three column slots (5 bits each, 31 = missing) */
   const uint64_t *batch_packed;    /* device, or NULL */
+  /* OP2HIP_ROWGATHER_TASKS (op2hip_task_plan_fill; cells and max_batch_cells
+     as there) */
+  const void *task_desc;           /* device, 16 int32 per batch */
+  const uint32_t *tasks;           /* device */
+  const uint16_t *task_multis;     /* device */
+  int32_t max_batch_multis;        /* largest count of blocks with several tasks */
 } op2hip_exec;
 
 /* Device CSR / BSR matrix on a fixed pattern (the reference's PETSc AIJ or
@@ -222,6 +234,29 @@ int op2hip_tile_targets_add(int32_t type, int32_t nrows, int32_t dim, const int3
 int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
                      const int32_t *rmap, int32_t rarity, const int32_t *cmap, int32_t carity,
                      int32_t *slots, int32_t *bad, void *stream);
+
+/* ---- task plan of OP2HIP_ROWGATHER_TASKS -------------------------------- */
+/* From row batches, their slot table's descriptors and a gather table
+ * (op2hip_gather_table_*): every output block's element blocks are cut into
+ * tasks of at most OP2HIP_TASK_LENGTH, longest tasks first in a batch.
+ * count: counts[3 * b + 0..2] = distinct elements, task words and blocks of
+ * several tasks of batch b, counts[3 * nbatches] the batches that do not fit
+ * (more than 512 elements, 1,024 incidences or 1,024 blocks).  fill, with the
+ * exclusive sums of the three: cells, their ascending element ids; multis,
+ * the blocks of several tasks; tasks, up to four words a task: its block (or
+ * 0x8000 + its place in multis) and its first code, then two codes each, a
+ * code being (element of the batch << 7) + i * carity + j; a batch's first
+ * words, then the second words of the tasks that have one, and so on; desc,
+ * per batch {z0, nz, first word, first cell, cells, first multi, multis, 0,
+ * tasks of at least 1..6 element blocks, 0, 0}.  rarity * carity at most 128. */
+int op2hip_task_plan_count(int32_t nbatches, const void *batch_desc, const uint8_t *gcount,
+                           const int32_t *inc_ent, int32_t rarity, int32_t *counts,
+                           void *stream);
+int op2hip_task_plan_fill(int32_t nbatches, const void *batch_desc, const uint8_t *gcount,
+                          const uint16_t *glist, const int32_t *inc_ent, int32_t rarity,
+                          int32_t carity, const int32_t *first_cell, const int32_t *first_word,
+                          const int32_t *first_multi, int32_t *cells, uint32_t *tasks,
+                          uint16_t *multis, void *desc, void *stream);
 
 /* ---- sparsity (replaces pyop2/sparsity.pyx:121-284, build_sparsity and
  *      fill_with_zeros, non-extruded, one DataSet pair) ------------------ */

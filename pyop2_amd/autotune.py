@@ -48,6 +48,10 @@ _loaded = False
 
 REPEATS = 5
 
+# Part of every decision's key: counts the changes of kernels or candidates, so
+# that a decision kept on disk by other ones is not taken up
+_KERNELS = 1
+
 # parameter candidates per strategy (the first is the strategy's default)
 STAGED_PARAMS = [
     {"tile": 256, "lds": 65536, "block": 256},
@@ -73,6 +77,13 @@ STAGED_COLOURED_PARAMS = [
 # write no matrix overlapped on a side stream, issued before / after the
 # assembly
 SPLIT_OVERLAP = [None, "before", "after"]
+# task row gathers: batches whose LDS lets four workgroups of 512 share a CU
+# (384 incidences / 480 blocks), or three with fewer, larger batches
+ROWGATHER_TASKS_PARAMS = [
+    {"batch": [384, 480], "block": 512},
+    {"batch": [576, 720], "block": 512},
+    {"batch": [192, 240], "block": 256},
+]
 ROWGATHER_PARAMS = {
     # P2 BSR(3) float64 / float32: (incidences, blocks) of a batch
     "p2": [{"batch": None, "block": 256},
@@ -122,8 +133,10 @@ def candidates(executor, parloop):
         if isinstance(parloop.iterset, Subset):
             return ["atomic", "coloured"]
         split = ["split"] if "split" in executor.spec else []
-        return split + ["rowgather_slots", "rowgather_rows", "rowgather_cells", "rowgather_staged",
-                        "rowgather_thread", "rowgather", "atomic"]
+        tasks = ["rowgather_tasks"] if executor.family == "p2_elasticity_matrix" else []
+        return split + ["rowgather_slots"] + tasks + ["rowgather_rows", "rowgather_cells",
+                                                       "rowgather_staged", "rowgather_thread",
+                                                       "rowgather", "atomic"]
     if "staged" in executor.spec and not isinstance(parloop.iterset, Subset):
         return ["staged", "staged_coloured", "atomic", "coloured"]
     return ["atomic", "coloured"]
@@ -135,6 +148,8 @@ def param_candidates(executor, strategy):
         return STAGED_PARAMS
     if strategy == "staged_coloured":
         return STAGED_COLOURED_PARAMS
+    if strategy == "rowgather_tasks":
+        return ROWGATHER_TASKS_PARAMS
     if strategy in ("rowgather_slots", "rowgather_rows"):
         return ROWGATHER_PARAMS["p2" if executor.family.startswith("p2_") else "p1"]
     return [{}]
@@ -161,7 +176,7 @@ def _key(executor, parloop):
     it = parloop.iterset
     maps = [map_digest(m) for a in parloop.arguments for m in a.maps]
     sub = it._plan_key()[-1] if isinstance(it, Subset) else None
-    return json.dumps([executor.family, executor.variant, type(it).__name__, it.core_size, it.size,
+    return json.dumps([_KERNELS, executor.family, executor.variant, type(it).__name__, it.core_size, it.size,
                        it.total_size, sub, maps])
 
 
@@ -253,7 +268,7 @@ def _time(executor, parloop, cfg, outputs, repeats):
 
 def _tune_split(executor, parloop, outputs, repeats, report):
     """Each part of a split loop tuned as a loop of its own (the assembly
-    part under the slot-table row gather; the other parts under each staged
+    part under the slot-table and task row gathers; the other parts under each staged
     strategy, partials and coloured tiles), on the split loop's scratch
     outputs.  The best configuration of every strategy of a part is kept:
     a part that is slower alone can be the faster one beside the assembly
@@ -270,24 +285,27 @@ def _tune_split(executor, parloop, outputs, repeats, report):
                 sub_out[n] = outputs[k]
         if "mat" in outputs:
             sub_out["mat"] = outputs["mat"]
-        wanted = (["rowgather_slots"] if sub.spec["args"][0][0] == "mat"
-                  else ["staged", "staged_coloured"])
-        strats = []
-        for w in wanted:
-            strat = sub.applicable(part, w)
-            if strat not in strats:
-                strats.append(strat)
-        alts = []
-        for strat in strats:
-            best, best_t = {"strategy": strat}, None
-            for params in param_candidates(sub, strat):
-                cfg = dict(params, strategy=strat)
-                t = _time(sub, part, cfg, sub_out, repeats)
-                if report is not None:
-                    report[f"{sub.family}:{json.dumps(cfg, sort_keys=True)}"] = t
-                if t is not None and (best_t is None or t < best_t):
-                    best, best_t = cfg, t
-            alts.append(best)
+        # the best of each group is kept: of the matrix, which takes most of
+        # the time, the one that is fastest alone
+        groups = ([["rowgather_slots", "rowgather_tasks"]] if sub.spec["args"][0][0] == "mat"
+                  else [["staged"], ["staged_coloured"]])
+        alts, seen = [], []
+        for group in groups:
+            best, best_t = None, None
+            for strat in dict.fromkeys(sub.applicable(part, w) for w in group):
+                if strat in seen:
+                    continue
+                seen.append(strat)
+                best = best or {"strategy": strat}
+                for params in param_candidates(sub, strat):
+                    cfg = dict(params, strategy=strat)
+                    t = _time(sub, part, cfg, sub_out, repeats)
+                    if report is not None:
+                        report[f"{sub.family}:{json.dumps(cfg, sort_keys=True)}"] = t
+                    if t is not None and (best_t is None or t < best_t):
+                        best, best_t = cfg, t
+            if best is not None:
+                alts.append(best)
         alternatives.append(alts)
     best, best_t = None, None
     for parts in itertools.product(*alternatives):

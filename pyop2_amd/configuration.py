@@ -29,7 +29,7 @@ _Option = namedtuple("_Option", "env type default")
 
 _STRATEGIES = frozenset(("auto", "atomic", "coloured", "staged", "staged_coloured", "split", "rowgather",
                          "rowgather_thread", "rowgather_slots", "rowgather_staged",
-                         "rowgather_cells", "rowgather_rows"))
+                         "rowgather_cells", "rowgather_rows", "rowgather_tasks"))
 
 
 def _from_env(opt):

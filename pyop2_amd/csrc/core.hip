@@ -1458,6 +1458,39 @@ int op2hip_plan_cell_gather(int32_t nbatches, const void *batch_desc, const void
   }
 }
 
+int op2hip_task_plan_count(int32_t nbatches, const void *batch_desc, const uint8_t *gcount,
+                           const int32_t *inc_ent, int32_t rarity, int32_t *counts,
+                           void *stream) {
+  hipStream_t s = stream_of(stream);
+  OP2HIP_REQUIRE(nbatches >= 0 && batch_desc && gcount && inc_ent && rarity > 0 && counts,
+                 "task_plan_count: bad arguments");
+  const int rc = fill(counts + 3 * (int64_t)nbatches, 1, 0, s);
+  if (rc || nbatches == 0) return rc;
+  task_plan_kernel<false><<<nbatches, 256, 0, s>>>(
+      nbatches, static_cast<const BatchDesc *>(batch_desc), gcount, nullptr, inc_ent, rarity, 1,
+      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, counts);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+int op2hip_task_plan_fill(int32_t nbatches, const void *batch_desc, const uint8_t *gcount,
+                          const uint16_t *glist, const int32_t *inc_ent, int32_t rarity,
+                          int32_t carity, const int32_t *first_cell, const int32_t *first_word,
+                          const int32_t *first_multi, int32_t *cells, uint32_t *tasks,
+                          uint16_t *multis, void *desc, void *stream) {
+  OP2HIP_REQUIRE(nbatches >= 0 && batch_desc && gcount && glist && inc_ent && rarity > 0 &&
+                     carity > 0 && rarity * carity <= 128 && first_cell && first_word &&
+                     first_multi && cells && tasks && multis && desc,
+                 "task_plan_fill: bad arguments");
+  if (nbatches == 0) return OP2HIP_OK;
+  task_plan_kernel<true><<<nbatches, 256, 0, stream_of(stream)>>>(
+      nbatches, static_cast<const BatchDesc *>(batch_desc), gcount, glist, inc_ent, rarity, carity,
+      first_cell, first_word, first_multi, cells, tasks, multis,
+      static_cast<TaskDesc *>(desc), nullptr);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
 int op2hip_gather_table_count(int32_t nbatches, int32_t batch_max_nnz, const void *batch_desc,
                               const void *table, int32_t carity, uint8_t *gcount,
                               int32_t *batch_total, int32_t *over, void *stream) {

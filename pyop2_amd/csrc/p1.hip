@@ -142,6 +142,7 @@ int op2hip_wrap_p1_laplace_matrix(int32_t start, int32_t end, const op2hip_mat *
     P1MatrixRow elem{X, c2v};
     return launch_rowgather(start, end, elem, A, ex, static_cast<double *>(nullptr), s);
   }
+  OP2HIP_REQUIRE(!ex || ex->strategy != OP2HIP_ROWGATHER_TASKS, "p1 matrix: no task row gather");
   const int bs = block_size_of(ex, 256);
   const op2hip_mat Av = *A;
   return for_each_launch(ex, start, end, [&](int32_t lo, int32_t hi, const int32_t *list,

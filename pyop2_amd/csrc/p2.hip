@@ -657,6 +657,104 @@ struct MatrixCells {
   }
 };
 
+// Task-gather element: per element the barycentric gradients gl[m] and
+// 0.8 wdet.  With basis i on the vertices (a, b) and j on (c, d) (b = a, d = c
+// for a vertex), sum_q grad phi_i (x) grad phi_j of the closed form above is
+//   0.8 ((x1 gl_a + x2 gl_b) (x) gl_c + (x3 gl_a + x4 gl_b) (x) gl_d)
+// with whole numbers x by the 100 pairs (i, j): the lookup table (the high
+// words of the doubles -1, 0, 3, 4, 8, whose low words are zero).  The block,
+// lam M + mu M^T + mu tr(M) I, is linear in M, so it is formed once per task.
+template <typename TT>
+struct MatrixTasks {
+  using T = TT;
+  static constexpr int kRar = 10, kCar = 10, kRd = 3, kCd = 3;
+  // 13 values a cell, padded to 28 words: successive cells start 28 banks on
+  static constexpr int kGeo = 14;
+  static constexpr int32_t kXcdChunk = 8;
+  static constexpr int kTableBytes = 100 * (16 + 4);
+  const T *X;
+  const int32_t *c2v;
+  T lam, mu;
+  __device__ __forceinline__ void geometry(int32_t e, double *geo) const {
+    double xv[4][3];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int32_t n = c2v[4 * e + v];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) xv[v][r] = double(X[3 * n + r]);
+    }
+    const Geom<double> g = geometry_of(xv);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) geo[3 * m + k] = g.gl[m][k];
+    geo[12] = 0.8 * g.wdet;
+  }
+  __device__ static __forceinline__ void no_geometry(double *geo) {
+#pragma unroll
+    for (int k = 0; k < 13; ++k) geo[k] = 0.0;
+  }
+  __device__ static __forceinline__ void fill_table(void *table) {
+    uint4 *x = static_cast<uint4 *>(table);
+    uint32_t *at = reinterpret_cast<uint32_t *>(x + 100);
+    for (int ij = threadIdx.x; ij < 100; ij += blockDim.x) {
+      const int i = ij / 10, j = ij - 10 * i;
+      int a, b, c, d;
+      MatrixCells<double, false>::ends(i, a, b);
+      MatrixCells<double, false>::ends(j, c, d);
+      constexpr uint32_t kM1 = 0xBFF00000u, k3 = 0x40080000u, k4 = 0x40100000u, k8 = 0x40200000u;
+      uint4 w = {0u, 0u, 0u, 0u};
+      if (i < 4 && j < 4) {
+        w.x = i == j ? k3 : kM1;
+      } else if (i < 4) {          // vertex row, edge column
+        w.x = d == i ? k3 : kM1;
+        w.z = c == i ? k3 : kM1;
+      } else if (j < 4) {          // edge row, vertex column
+        w.x = j == b ? k3 : kM1;
+        w.y = j == a ? k3 : kM1;
+      } else {
+        w.x = d == b ? k8 : k4;
+        w.y = d == a ? k8 : k4;
+        w.z = c == b ? k8 : k4;
+        w.w = c == a ? k8 : k4;
+      }
+      x[ij] = w;
+      at[ij] = a | b << 8 | c << 16 | d << 24;
+    }
+  }
+  __device__ static __forceinline__ void add(const double *geo, int ij, const void *table,
+                                             double *M) {
+    const uint4 w = static_cast<const uint4 *>(table)[ij];
+    const uint32_t at = reinterpret_cast<const uint32_t *>(static_cast<const uint4 *>(table) + 100)[ij];
+    const double *ga = geo + 3 * (at & 255u), *gb = geo + 3 * (at >> 8 & 255u),
+                 *gc = geo + 3 * (at >> 16 & 255u), *gd = geo + 3 * (at >> 24);
+    const double s = geo[12];
+    const double x1 = s * __hiloint2double((int)w.x, 0), x2 = s * __hiloint2double((int)w.y, 0);
+    const double x3 = s * __hiloint2double((int)w.z, 0), x4 = s * __hiloint2double((int)w.w, 0);
+    double P[3], Q[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      P[k] = x1 * ga[k] + x2 * gb[k];
+      Q[k] = x3 * ga[k] + x4 * gb[k];
+    }
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const double c = gc[l], d = gd[l];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) M[3 * k + l] += P[k] * c + Q[k] * d;
+    }
+  }
+  __device__ __forceinline__ void finish(const double *M, double *B) const {
+    const double l = double(lam), m = double(mu);
+    const double tr = m * (M[0] + M[4] + M[8]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b)
+        B[3 * a + b] = l * M[3 * a + b] + m * M[3 * b + a] + (a == b ? tr : 0.0);
+  }
+};
+
 // Lane-per-block row-gather element: lane j of a group computes block (i, j).
 template <typename TT, bool kFused>
 struct MatrixLanes {
@@ -1001,6 +1099,10 @@ int matrix(int32_t start, int32_t end, const op2hip_mat *A, T *R, const T *X, co
   if (ex && ex->strategy == OP2HIP_ROWGATHER_CELLS) {
     MatrixCells<T, kFused> elem{X, u, c2v, T(lam), T(mu)};
     return launch_rowgather_cells(start, end, elem, A, ex, R, s);
+  }
+  if (ex && ex->strategy == OP2HIP_ROWGATHER_TASKS) {
+    OP2HIP_REQUIRE(!kFused, "the fused loop has no task row gather");
+    return launch_rowgather_tasks(start, end, MatrixTasks<T>{X, c2v, T(lam), T(mu)}, A, ex, s);
   }
   if (ex && ex->strategy == OP2HIP_ROWGATHER_THREAD) {
     MatrixRow<T, kFused> elem{X, u, c2n, c2v, T(lam), T(mu)};

@@ -1309,6 +1309,604 @@ int launch_rowgather_cells(int32_t start, int32_t end, const Elem &elem, const o
 }
 
 // ---------------------------------------------------------------------------
+// Task row gather.  The slot-table gather adds every element block into LDS, nine
+// float64 atomics a block (492 million for the 45^3 cube), and keeps float32
+// values in LDS as float64: its workgroups are few and wait.  Here an
+// element's geometry is staged in LDS once per batch, and a lane adds the
+// element blocks of one output block up in registers: at most kTaskLength of
+// them (a task), so that a wave's lanes stay together (tasks are sorted by
+// length) and the blocks that many elements share (the diagonal blocks of
+// vertices) do not keep one lane busy long after the others.  A block with one
+// task is added to the batch's values in LDS by its lane alone; the few with
+// several go through float64 sums of their own.
+//
+// What bounds it: the chain of a batch -- descriptor, elements, vertices,
+// coordinates, tasks, each a dependent access -- against how many batches a CU
+// holds, so small registers (64: eight waves a SIMD) and small LDS matter most:
+// 45^3 float32 in batches of 480 blocks and 512 threads, four workgroups a CU,
+// 421 us (545 with the slot table; without elements' work 320, at which rate
+// the values stream); with 69 registers and three workgroups 488; requests one
+// batch ahead in a persistent workgroup (128 registers) 472; values read
+// and written by the task lanes without LDS 500.  float64 takes 676 against
+// 622 us with the slot table (twice the LDS a block), so the tuner keeps that
+// for most of its sizes.
+//
+// Elem must additionally provide
+//   static constexpr int kGeo;                          // even
+//   void geometry(int32_t e, double *geo) const;        // kGeo doubles
+//   static void no_geometry(double *geo);               // element adds zero blocks
+//   void block(const double *geo, int i, int j, T *blk) const;  // runtime i, j
+//   void rowdat(int32_t col, const T *blk, Acc *rs) const;      // fused rows only
+
+template <class Elem>
+struct CellsLayout {
+  // region A holds the staged geometry, then (after the blocks are summed) the
+  // batch's new block values for the coalesced flush
+  __host__ __device__ static size_t region_a(int32_t max_cells, int32_t max_nnz) {
+    const size_t g = (size_t)max_cells * Elem::kGeo * sizeof(double);
+    const size_t r = (size_t)max_nnz * Elem::kRd * Elem::kCd * sizeof(double);
+    return ((g > r ? g : r) + 15) & ~(size_t)15;
+  }
+  static size_t bytes(int32_t max_cells, int32_t max_nnz, int32_t max_contrib, int32_t max_rows,
+                      int kOut) {
+    size_t b = region_a(max_cells, max_nnz);
+    b += (((size_t)max_contrib * sizeof(uint16_t)) + 15) & ~(size_t)15;
+    b += (size_t)kOut * 4 * sizeof(int32_t);
+    if (Elem::kHasRowDat)
+      b += (size_t)(max_rows + 2) * sizeof(int32_t) + (size_t)max_rows * Elem::kRd * sizeof(double);
+    return b;
+  }
+};
+
+template <class Elem, int kOut, int kPre>
+__global__ void __launch_bounds__(256)
+rowgather_cells_kernel(int32_t start, int32_t end, Elem elem, op2hip_mat A,
+                       const BatchDesc *__restrict__ descs, int32_t nbatches,
+                       const int32_t *__restrict__ cell_ptr, const int32_t *__restrict__ cells,
+                       const uint8_t *__restrict__ gcount, const uint16_t *__restrict__ order,
+                       const int32_t *__restrict__ contrib_ptr,
+                       const uint16_t *__restrict__ contrib, int32_t max_cells, int32_t max_nnz,
+                       int32_t max_contrib, typename Elem::T *__restrict__ rowdat) {
+  using T = typename Elem::T;
+  using Acc = typename AccumOf<T>::type;
+  constexpr int kBs = Elem::kRd * Elem::kCd;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+  const int32_t b = xcd_contiguous(blockIdx.x, nbatches);
+  const BatchDesc d = descs[b];
+  const int32_t c0 = cell_ptr[b], nc = cell_ptr[b + 1] - c0;
+  const int32_t g0 = contrib_ptr[b], ng = contrib_ptr[b + 1] - g0;
+  T *__restrict__ vals = static_cast<T *>(A.values) + (size_t)d.z0 * kBs;
+  const int32_t nval = d.nz * kBs;
+
+  double *geo = reinterpret_cast<double *>(smem);
+  double *res = geo;  // region A, reused after the sums
+  size_t off = CellsLayout<Elem>::region_a(max_cells, max_nnz);
+  uint16_t *clist = reinterpret_cast<uint16_t *>(smem + off);
+  off += (((size_t)max_contrib * sizeof(uint16_t)) + 15) & ~(size_t)15;
+  int32_t *wtot = reinterpret_cast<int32_t *>(smem + off);
+  off += (size_t)kOut * 4 * sizeof(int32_t);
+  int32_t *srow = reinterpret_cast<int32_t *>(smem + off);
+  double *racc = reinterpret_cast<double *>(
+      smem + off + (((size_t)(d.nr + 1) * sizeof(int32_t) + 7) & ~(size_t)7));
+
+  // old values of the batch, coalesced, in flight during the element work
+  T old[kPre];
+#pragma unroll
+  for (int u = 0; u < kPre; ++u) {
+    const int32_t k = threadIdx.x + u * (int32_t)blockDim.x;
+    old[u] = k < nval ? vals[k] : T(0);
+  }
+  int32_t z[kOut], cnt[kOut];
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    const int32_t w = threadIdx.x + o * (int32_t)blockDim.x;
+    z[o] = w < d.nz ? int32_t(order[(size_t)d.z0 + w]) : 0;
+    cnt[o] = w < d.nz ? int32_t(gcount[(size_t)d.z0 + z[o]]) : 0;
+  }
+  for (int32_t k = threadIdx.x; k < ng; k += blockDim.x) clist[k] = contrib[(size_t)g0 + k];
+  if (Elem::kHasRowDat) {
+    for (int32_t k = threadIdx.x; k <= d.nr; k += blockDim.x) srow[k] = A.rowptr[d.r0 + k] - d.z0;
+    for (int32_t k = threadIdx.x; k < d.nr * Elem::kRd; k += blockDim.x) racc[k] = 0.0;
+  }
+  for (int32_t u = threadIdx.x; u < nc; u += blockDim.x) {
+    const int32_t e = cells[(size_t)c0 + u];
+    if (e >= start && e < end) elem.geometry(e, geo + (size_t)u * Elem::kGeo);
+    else Elem::no_geometry(geo + (size_t)u * Elem::kGeo);
+  }
+
+  // exclusive scan of the counts in thread order
+  int32_t incl[kOut];
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    int32_t x = cnt[o];
+#pragma unroll
+    for (int dd = 1; dd < 64; dd <<= 1) {
+      const int32_t y = __shfl_up(x, dd, 64);
+      if (lane >= dd) x += y;
+    }
+    incl[o] = x;
+    if (lane == 63) wtot[o * 4 + wave] = x;
+  }
+  __syncthreads();
+
+  Acc acc[kOut][kBs];
+  int32_t base = 0;
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    int32_t before = 0, all = 0;
+    for (int w = 0; w < nwaves; ++w) {
+      const int32_t v = wtot[o * 4 + w];
+      before += w < wave ? v : 0;
+      all += v;
+    }
+    const int32_t first = base + before + incl[o] - cnt[o];
+    base += all;
+#pragma unroll
+    for (int k = 0; k < kBs; ++k) acc[o][k] = Acc(0);
+    for (int32_t c = 0; c < cnt[o]; ++c) {
+      const uint32_t code = clist[first + c];
+      T blk[kBs];
+      elem.block(geo + (size_t)(code >> 8) * Elem::kGeo, int((code >> 4) & 15u), int(code & 15u),
+                 blk);
+#pragma unroll
+      for (int k = 0; k < kBs; ++k) acc[o][k] += Acc(blk[k]);
+    }
+  }
+  __syncthreads();  // geometry no longer needed: region A takes the sums
+
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    const int32_t w = threadIdx.x + o * (int32_t)blockDim.x;
+    if (w >= d.nz) continue;
+#pragma unroll
+    for (int k = 0; k < kBs; ++k) res[(size_t)z[o] * kBs + k] = acc[o][k];
+    if (Elem::kHasRowDat) {
+      // the row's residual gets this block's new contribution times u[col]
+      int32_t lo = 0, hi = d.nr;
+      while (hi - lo > 1) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (srow[mid] <= z[o]) lo = mid; else hi = mid;
+      }
+      T add[kBs];
+#pragma unroll
+      for (int k = 0; k < kBs; ++k) add[k] = T(acc[o][k]);
+      Acc rs[Elem::kRd];
+#pragma unroll
+      for (int a = 0; a < Elem::kRd; ++a) rs[a] = Acc(0);
+      elem.rowdat(A.colidx[(size_t)d.z0 + z[o]], add, rs);
+#pragma unroll
+      for (int a = 0; a < Elem::kRd; ++a) atomic_add(&racc[lo * Elem::kRd + a], rs[a]);
+    }
+  }
+  __syncthreads();
+
+#pragma unroll
+  for (int u = 0; u < kPre; ++u) {
+    const int32_t k = threadIdx.x + u * (int32_t)blockDim.x;
+    if (k < nval) vals[k] = old[u] + T(res[k]);
+  }
+  for (int32_t k0 = threadIdx.x + kPre * (int32_t)blockDim.x; k0 < nval; k0 += 8 * (int32_t)blockDim.x) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int32_t k = k0 + u * (int32_t)blockDim.x;
+      v[u] = k < nval ? vals[k] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int32_t k = k0 + u * (int32_t)blockDim.x;
+      if (k < nval) vals[k] = v[u] + T(res[k]);
+    }
+  }
+  if (Elem::kHasRowDat) {
+    T *rd = rowdat + (size_t)d.r0 * Elem::kRd;
+    for (int32_t k = threadIdx.x; k < d.nr * Elem::kRd; k += blockDim.x) rd[k] += T(racc[k]);
+  }
+}
+
+template <class Elem>
+int launch_rowgather_cells(int32_t start, int32_t end, const Elem &elem, const op2hip_mat *A,
+                           const op2hip_exec *ex, typename Elem::T *rowdat, hipStream_t s) {
+  OP2HIP_REQUIRE(ex && ex->batch_desc && ex->cell_ptr && ex->cells && ex->gather_count &&
+                     ex->block_order && ex->contrib_ptr && ex->contrib && ex->nbatches >= 0,
+                 "cell-gather row gather without its plan");
+  OP2HIP_REQUIRE(!ex->subset, "row-gather assembly does not iterate Subsets");
+  OP2HIP_REQUIRE(A->rdim == Elem::kRd && A->cdim == Elem::kCd,
+                 "matrix block %dx%d, kernel assembles %dx%d", A->rdim, A->cdim,
+                 Elem::kRd, Elem::kCd);
+  if (end <= start || ex->nbatches == 0) return OP2HIP_OK;
+  const int bs = block_size_of(ex, 256);
+  OP2HIP_REQUIRE(bs > 0 && bs <= 256 && bs % 64 == 0, "row-gather block size %d", bs);
+  OP2HIP_REQUIRE(ex->max_batch_cells > 0 && ex->max_batch_cells <= 256 && ex->max_batch_contrib >= 0,
+                 "cell-gather plan: bad maxima");
+  const int32_t nout = (ex->batch_max_nnz + bs - 1) / bs;
+  OP2HIP_REQUIRE(nout <= 4, "cell-gather row gather: %d blocks in a batch, at most %d",
+                 ex->batch_max_nnz, 4 * bs);
+  const int kout = nout <= 1 ? 1 : (nout <= 2 ? 2 : 4);
+  const size_t lds = CellsLayout<Elem>::bytes(ex->max_batch_cells, ex->batch_max_nnz,
+                                              ex->max_batch_contrib, ex->batch_max_rows, kout);
+  OP2HIP_REQUIRE(lds <= 64 * 1024, "row batch needs %zu bytes of LDS (max 65536)", lds);
+  const auto *descs = static_cast<const BatchDesc *>(ex->batch_desc);
+  // prefetch depth: the batch's values per thread, at most 24
+  const int64_t per_thread = ((int64_t)ex->batch_max_nnz * Elem::kRd * Elem::kCd + bs - 1) / bs;
+#define OP2HIP_CELLS(K, P)                                                                     \
+  rowgather_cells_kernel<Elem, K, P><<<ex->nbatches, bs, lds, s>>>(                            \
+      start, end, elem, *A, descs, ex->nbatches, ex->cell_ptr, ex->cells, ex->gather_count,    \
+      ex->block_order, ex->contrib_ptr, ex->contrib, ex->max_batch_cells, ex->batch_max_nnz,   \
+      ex->max_batch_contrib, rowdat)
+  if (per_thread <= 8) {
+    if (kout == 1) OP2HIP_CELLS(1, 8);
+    else if (kout == 2) OP2HIP_CELLS(2, 8);
+    else OP2HIP_CELLS(4, 8);
+  } else if (per_thread <= 16) {
+    if (kout == 1) OP2HIP_CELLS(1, 16);
+    else if (kout == 2) OP2HIP_CELLS(2, 16);
+    else OP2HIP_CELLS(4, 16);
+  } else {
+    if (kout == 1) OP2HIP_CELLS(1, 24);
+    else if (kout == 2) OP2HIP_CELLS(2, 24);
+    else OP2HIP_CELLS(4, 24);
+  }
+#undef OP2HIP_CELLS
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Task row gather.  LDS float64 atomic adds run at about one a clock and CU, so
+// a batch that adds every element block into LDS (nine adds a block, the
+// slot-table gather) is bound by them: 583 us for the 45^3 float32 assembly
+// whose values take 265 us to stream.  Here an element's geometry is staged in
+// LDS once per batch, and a lane adds the element blocks of one output block up
+// in registers: at most kTaskLength of them (a task), so that a wave's lanes
+// stay together (tasks are sorted by length) and the blocks that many elements
+// share (the diagonal blocks of vertices) do not keep one lane busy long after
+// the others.  A block with one task is added to the batch's values in LDS by
+// its lane alone; the few with several go through float64 sums of their own.
+//
+// Elem must additionally provide
+//   static constexpr int kGeo;                       doubles of geometry an element
+//   void geometry(int32_t e, double *geo) const;
+//   static void no_geometry(double *geo);            element adds zero blocks
+//   static constexpr int kTableBytes;                lookup table in LDS, by row and column
+//   static void fill_table(void *table);             all threads of the workgroup
+//   static void add(const double *geo, int ij, const void *table, double *sum);
+//   void finish(const double *sum, double *blk) const;   linear in sum
+constexpr int kTaskLength = OP2HIP_TASK_LENGTH;
+
+// A task is up to four 32-bit words: its output block (or 0x8000 + its place
+// among the blocks of several tasks) and first code, then its codes two by
+// two; the first words of all tasks of a batch, the second words of those that
+// have one, and so on, so that a wave's loads are whole lines.
+struct TaskDesc {
+  int32_t z0, nz, word0, cell0, ncell, multi0, nmulti, pad0;
+  int32_t n[kTaskLength];   // tasks of at least 1, 2, ... element blocks
+  int32_t pad1[2];
+};
+constexpr int kTaskWords = kTaskLength / 2 + 1;
+// the element blocks a task must have for its word u
+__host__ __device__ constexpr int task_word_from(int u) { return u == 0 ? 1 : 2 * u; }
+static_assert(sizeof(TaskDesc) == 64, "sixteen words a batch");
+
+template <class Elem>
+struct TaskLayout {
+  using T = typename Elem::T;
+  static constexpr int kBs = Elem::kRd * Elem::kCd;
+  // the values, and a 16-byte word before and behind them (see the kernel)
+  __host__ __device__ static size_t geo_at(int32_t max_nnz) {
+    return ((size_t)max_nnz * kBs * sizeof(T) + 47) & ~(size_t)15;
+  }
+  __host__ __device__ static size_t multi_at(int32_t max_nnz, int32_t max_cells) {
+    return geo_at(max_nnz) + (size_t)max_cells * Elem::kGeo * sizeof(double);
+  }
+  __host__ __device__ static size_t table_at(int32_t max_nnz, int32_t max_cells, int32_t max_multis) {
+    return (multi_at(max_nnz, max_cells) + (size_t)max_multis * kBs * sizeof(double) + 15) & ~(size_t)15;
+  }
+  static size_t bytes(int32_t max_nnz, int32_t max_cells, int32_t max_multis) {
+    return table_at(max_nnz, max_cells, max_multis) + Elem::kTableBytes;
+  }
+};
+
+// 16 bytes of values: the unit the task gather moves them in.
+template <typename T>
+struct ValueWord {
+  static constexpr int kN = 16 / sizeof(T);
+  typedef T type __attribute__((ext_vector_type(kN)));
+};
+
+// Where a batch's values lie: `head` values before the first 16-byte boundary,
+// then whole words, then the rest.  In LDS word k lies at slot 1 + k, the head
+// at the end of slot 0.
+template <typename T, int kBs>
+struct BatchValues {
+  using W = typename ValueWord<T>::type;
+  static constexpr int kW = ValueWord<T>::kN;
+  T *vals;
+  int32_t nval, head, nword;
+  __device__ __forceinline__ BatchValues(T *values, int32_t z0, int32_t nz)
+      : vals(values + (size_t)z0 * kBs), nval(nz * kBs) {
+    const int32_t off = (int32_t)(reinterpret_cast<uintptr_t>(vals) & 15) / (int32_t)sizeof(T);
+    head = min(nval, (kW - off) & (kW - 1));
+    nword = (nval - head) / kW;
+  }
+  __device__ __forceinline__ W *words() const { return reinterpret_cast<W *>(vals + head); }
+};
+
+template <class Elem>
+__global__ void __launch_bounds__(512, 8)
+rowgather_tasks_kernel(int32_t start, int32_t end, Elem elem, op2hip_mat A,
+                       const TaskDesc *__restrict__ descs, int32_t nbatches,
+                       const int32_t *__restrict__ cells, const uint32_t *__restrict__ tasks,
+                       const uint16_t *__restrict__ multis, int32_t max_nnz, int32_t max_cells,
+                       int32_t max_multis) {
+  using T = typename Elem::T;
+  using L = TaskLayout<Elem>;
+  constexpr int kBs = L::kBs;
+  using V = BatchValues<T, kBs>;
+  using W = typename V::W;
+  constexpr int kW = V::kW;
+  constexpr int kDepth = 4;   // words of old values in flight per thread
+  extern __shared__ __align__(16) unsigned char smem[];
+  W *slots = reinterpret_cast<W *>(smem) + 1;
+  double *geo = reinterpret_cast<double *>(smem + L::geo_at(max_nnz));
+  double *multi = reinterpret_cast<double *>(smem + L::multi_at(max_nnz, max_cells));
+  void *table = smem + L::table_at(max_nnz, max_cells, max_multis);
+  const TaskDesc &d = descs[xcd_dealt<XcdChunkOf<Elem>::value>(blockIdx.x, nbatches)];
+  const V v(static_cast<T *>(A.values), d.z0, d.nz);
+  T *acc = reinterpret_cast<T *>(slots) - v.head;
+  W *words = v.words();
+  const int32_t bd = (int32_t)blockDim.x, tail = v.head + v.nword * kW;
+  // Tasks are sorted by length and elements fill the first waves only: which
+  // wave takes which part of either turns with the batch, or the SIMD that
+  // gets every workgroup's first wave would hold the others up.
+  const int32_t turn = (int32_t)(blockIdx.x / 8) % (bd / 64) * 64;
+  const int32_t mine = ((int32_t)threadIdx.x + turn) % bd;
+  const int32_t cell = bd - 64 - (mine & ~63) + (mine & 63);
+  // the thread's first element and task before the bulk of the old values
+  const int32_t e0 = cell < d.ncell ? cells[d.cell0 + cell] : -1;
+  uint32_t task[kTaskWords];
+  auto load_task = [&](int32_t t) {
+    const uint32_t *p = tasks + d.word0 + t;
+#pragma unroll
+    for (int u = 0; u < kTaskWords; ++u) {
+      const int32_t n = d.n[task_word_from(u) - 1];
+      if (t < n) task[u] = __builtin_nontemporal_load(p);
+      p += n;
+    }
+  };
+  load_task(mine);
+  Elem::fill_table(table);
+  for (int32_t k = threadIdx.x; k < d.nmulti * kBs; k += bd) multi[k] = 0.0;
+  for (int32_t u = cell; u < d.ncell; u += bd) {
+    const int32_t e = u == cell ? e0 : cells[d.cell0 + u];
+    double *g = geo + (size_t)u * Elem::kGeo;
+    if (e >= start && e < end) elem.geometry(e, g);
+    else Elem::no_geometry(g);
+  }
+  for (int32_t k0 = threadIdx.x; k0 < v.nword; k0 += kDepth * bd) {
+    W w[kDepth];
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u)
+      if (k0 + u * bd < v.nword) w[u] = __builtin_nontemporal_load(&words[k0 + u * bd]);
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u)
+      if (k0 + u * bd < v.nword) slots[k0 + u * bd] = w[u];
+  }
+  if ((int32_t)threadIdx.x < v.head) acc[threadIdx.x] = v.vals[threadIdx.x];
+  if (tail + (int32_t)threadIdx.x < v.nval) acc[tail + threadIdx.x] = v.vals[tail + threadIdx.x];
+  __syncthreads();
+
+  for (int32_t t = mine; t < d.n[0]; t += bd) {
+    if (t != mine) load_task(t);
+    double sum[kBs];
+#pragma unroll
+    for (int k = 0; k < kBs; ++k) sum[k] = 0.0;
+#pragma unroll
+    for (int u = 0; u < kTaskLength; ++u) {
+      if (t >= d.n[u]) break;
+      const uint32_t pair = task[(u + 1) / 2];
+      const uint32_t code = u % 2 ? pair & 0xffffu : pair >> 16;
+      Elem::add(geo + (size_t)(code >> 7) * Elem::kGeo, code & 127, table, sum);
+    }
+    double blk[kBs];
+    elem.finish(sum, blk);
+    const uint32_t to = task[0] & 0xffffu;
+    if (to < 0x8000u) {
+      T *out = acc + (size_t)to * kBs;
+#pragma unroll
+      for (int k = 0; k < kBs; ++k) out[k] += T(blk[k]);
+    } else {
+      double *out = multi + (size_t)(to & 0x7fffu) * kBs;
+#pragma unroll
+      for (int k = 0; k < kBs; ++k) atomic_add(&out[k], blk[k]);
+    }
+  }
+  __syncthreads();
+  if (d.nmulti > 0) {
+    for (int32_t k = threadIdx.x; k < d.nmulti * kBs; k += bd) {
+      const int32_t m = k / kBs;
+      acc[(size_t)multis[d.multi0 + m] * kBs + (k - m * kBs)] += T(multi[k]);
+    }
+    __syncthreads();
+  }
+  for (int32_t k = threadIdx.x; k < v.nword; k += bd) __builtin_nontemporal_store(slots[k], &words[k]);
+  if ((int32_t)threadIdx.x < v.head) v.vals[threadIdx.x] = acc[threadIdx.x];
+  if (tail + (int32_t)threadIdx.x < v.nval) v.vals[tail + threadIdx.x] = acc[tail + threadIdx.x];
+}
+
+template <class Elem>
+int launch_rowgather_tasks(int32_t start, int32_t end, const Elem &elem, const op2hip_mat *A,
+                           const op2hip_exec *ex, hipStream_t s) {
+  OP2HIP_REQUIRE(ex && ex->task_desc && ex->tasks && ex->task_multis && ex->cells &&
+                     ex->nbatches >= 0 && ex->max_batch_cells >= 0 && ex->max_batch_multis >= 0,
+                 "task row gather without its plan");
+  OP2HIP_REQUIRE(!ex->subset, "row-gather assembly does not iterate Subsets");
+  OP2HIP_REQUIRE(A->rdim == Elem::kRd && A->cdim == Elem::kCd,
+                 "matrix block %dx%d, kernel assembles %dx%d", A->rdim, A->cdim,
+                 Elem::kRd, Elem::kCd);
+  if (end <= start || ex->nbatches == 0) return OP2HIP_OK;
+  const size_t lds =
+      TaskLayout<Elem>::bytes(ex->batch_max_nnz, ex->max_batch_cells, ex->max_batch_multis);
+  OP2HIP_REQUIRE(lds <= 64 * 1024, "row batch needs %zu bytes of LDS (max 65536)", lds);
+  const int bs = block_size_of(ex, 512);
+  OP2HIP_REQUIRE(bs > 0 && bs <= 512 && bs % 64 == 0, "row-gather block size %d", bs);
+  rowgather_tasks_kernel<Elem><<<ex->nbatches, bs, lds, s>>>(
+      start, end, elem, *A, static_cast<const TaskDesc *>(ex->task_desc), ex->nbatches, ex->cells,
+      ex->tasks, ex->task_multis, ex->batch_max_nnz, ex->max_batch_cells, ex->max_batch_multis);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+// Task plan kernels, one workgroup a batch: the distinct elements by a hash
+// table in LDS, ranked; every output block's element blocks (its run of the
+// gather list, in incidence order) cut into tasks of nearly equal length; the
+// tasks of each length numbered in block order.
+constexpr int kTaskMaxInc = 1024, kTaskMaxCells = 512;
+
+template <bool kFill>
+__global__ void __launch_bounds__(256)
+task_plan_kernel(int32_t nbatches, const BatchDesc *__restrict__ batches,
+                 const uint8_t *__restrict__ gcount, const uint16_t *__restrict__ glist,
+                 const int32_t *__restrict__ inc_ent, int32_t rarity, int32_t carity,
+                 const int32_t *__restrict__ first_cell, const int32_t *__restrict__ first_word,
+                 const int32_t *__restrict__ first_multi, int32_t *__restrict__ cells,
+                 uint32_t *__restrict__ tasks, uint16_t *__restrict__ multis,
+                 TaskDesc *__restrict__ desc,
+                 int32_t *__restrict__ counts) {
+  constexpr int kSlots = 2 * kTaskMaxInc;
+  __shared__ int32_t keys[kSlots];
+  __shared__ int32_t found[kTaskMaxInc], sorted[kTaskMaxInc];
+  __shared__ int32_t ncell, bad;
+  __shared__ uint8_t cnt[kGatherMaxBlocks];
+  __shared__ uint16_t run[kGatherMaxBlocks], at_long[kGatherMaxBlocks], at_short[kGatherMaxBlocks],
+      mult[kGatherMaxBlocks];
+  __shared__ int32_t n_of[kTaskLength + 1], base_of[kTaskLength + 1], off_of[kTaskWords];
+  __shared__ int32_t nmulti;
+  const int32_t b = blockIdx.x;
+  if (b >= nbatches) return;
+  const BatchDesc d = batches[b];
+  if (threadIdx.x == 0) {
+    ncell = 0;
+    bad = d.ni > kTaskMaxInc || d.nz > kGatherMaxBlocks;
+  }
+  for (int k = threadIdx.x; k < kSlots; k += 256) keys[k] = -1;
+  __syncthreads();
+  if (bad) {
+    if (!kFill && threadIdx.x == 0) {
+      counts[3 * b] = counts[3 * b + 1] = counts[3 * b + 2] = 0;
+      atomicAdd(&counts[3 * (int64_t)nbatches], 1);
+    }
+    return;
+  }
+  for (int32_t z = threadIdx.x; z < d.nz; z += 256) cnt[z] = gcount[(size_t)d.z0 + z];
+  for (int32_t t = threadIdx.x; t < d.ni; t += 256) {
+    const int32_t e = inc_ent[d.i0 + t] / rarity;
+    uint32_t h = ((uint32_t)e * 2654435761u) / (uint32_t)(0x100000000ull / kSlots);
+    for (;;) {   // ends: at most half the slots are taken
+      const int32_t was = atomicCAS(&keys[h], -1, e);
+      if (was == -1) found[atomicAdd(&ncell, 1)] = e;
+      if (was == -1 || was == e) break;
+      h = (h + 1) & (kSlots - 1);
+    }
+  }
+  __syncthreads();
+  const int32_t nc = ncell;
+  auto tasks_of = [](int32_t c) { return (c + kTaskLength - 1) / kTaskLength; };
+  // threads 1..kTaskLength number the tasks of their length, thread 0 the
+  // blocks' runs and the blocks of several tasks
+  if (threadIdx.x == 0) {
+    int32_t r = 0, m = 0;
+    for (int32_t z = 0; z < d.nz; ++z) {
+      run[z] = (uint16_t)r;
+      mult[z] = (uint16_t)m;
+      r += cnt[z];
+      m += cnt[z] > kTaskLength;
+    }
+    nmulti = m;
+  } else if (threadIdx.x <= kTaskLength) {
+    const int32_t len = threadIdx.x;
+    int32_t n = 0;
+    for (int32_t z = 0; z < d.nz; ++z) {
+      const int32_t c = cnt[z], nt = tasks_of(c);
+      if (nt == 0) continue;
+      const int32_t lo = c / nt, more = c - lo * nt;   // `more` tasks of lo + 1, the rest of lo
+      if (lo + 1 == len && more) { at_long[z] = (uint16_t)n; n += more; }
+      if (lo == len) { at_short[z] = (uint16_t)n; n += nt - more; }
+    }
+    n_of[len] = n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t at = 0;
+    for (int len = kTaskLength; len >= 1; --len) {
+      base_of[len] = at;
+      at += n_of[len];
+    }
+    int32_t off = 0;
+    for (int u = 0; u < kTaskWords; ++u) {   // longer tasks come first
+      off_of[u] = off;
+      off += base_of[task_word_from(u)] + n_of[task_word_from(u)];
+    }
+    if constexpr (!kFill) {
+      counts[3 * b] = nc;
+      counts[3 * b + 1] = off;
+      counts[3 * b + 2] = nmulti;
+      if (nc > kTaskMaxCells) atomicAdd(&counts[3 * (int64_t)nbatches], 1);
+    } else {
+      TaskDesc &o = desc[b];
+      o.z0 = d.z0;
+      o.nz = d.nz;
+      o.word0 = first_word[b];
+      o.cell0 = first_cell[b];
+      o.ncell = nc;
+      o.multi0 = first_multi[b];
+      o.nmulti = nmulti;
+      for (int u = 0; u < kTaskLength; ++u) o.n[u] = base_of[u + 1] + n_of[u + 1];
+      o.pad0 = o.pad1[0] = o.pad1[1] = 0;
+    }
+  }
+  if constexpr (kFill) {
+    __syncthreads();
+    for (int32_t k = threadIdx.x; k < nc; k += 256) {
+      int32_t rank = 0;
+      for (int32_t t = 0; t < nc; ++t) rank += found[t] < found[k];
+      sorted[rank] = found[k];
+    }
+    __syncthreads();
+    for (int32_t k = threadIdx.x; k < nc; k += 256) cells[(size_t)first_cell[b] + k] = sorted[k];
+    for (int32_t z = threadIdx.x; z < d.nz; z += 256) {
+      const int32_t c = cnt[z], nt = tasks_of(c);
+      if (nt == 0) continue;
+      const int32_t lo = c / nt, more = c - lo * nt;
+      if (nt > 1) multis[(size_t)first_multi[b] + mult[z]] = (uint16_t)z;
+      const uint16_t word = nt > 1 ? (uint16_t)(0x8000 | mult[z]) : (uint16_t)z;
+      const uint16_t *list = glist + (size_t)d.pad0 + run[z];
+      int32_t q = 0;
+      for (int32_t k = 0; k < nt; ++k) {
+        const int32_t len = lo + (k < more);
+        const int32_t tau = base_of[len] + (k < more ? at_long[z] + k : at_short[z] + k - more);
+        uint32_t pair = word;
+        for (int32_t u = 0; u < len; ++u, ++q) {
+          const int32_t t = list[q] / carity, j = list[q] - t * carity;
+          const int32_t ent = inc_ent[d.i0 + t], e = ent / rarity;
+          int32_t x = 0, y = nc - 1;
+          while (x < y) {
+            const int32_t mid = (x + y) >> 1;
+            if (sorted[mid] < e) x = mid + 1; else y = mid;
+          }
+          const uint32_t code = (uint32_t)(x << 7 | ((ent - e * rarity) * carity + j));
+          if (u % 2) pair = code;
+          else pair |= code << 16;
+          tasks[(size_t)first_word[b] + off_of[(u + 1) / 2] + tau] = pair;
+          if (u % 2 == 0) pair = 0;
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Row-list row gather: the slot-table row gather over batches of rows taken
 // in an element-local order (op2hip_plan_row_list) rather than consecutive
 // row ids.  With a scattered row numbering (a permuted mesh) a batch of

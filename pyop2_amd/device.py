@@ -21,12 +21,12 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "li
 
 OK, ERR_HIP, ERR_ARG, ERR_WORKSPACE, ERR_OVERFLOW, ERR_JIT, ERR_PATTERN = range(7)
 (ATOMIC, COLOURED, STAGED, ROWGATHER, ROWGATHER_THREAD, ROWGATHER_SLOTS, ROWGATHER_STAGED,
- ROWGATHER_CELLS, ROWGATHER_ROWLIST) = range(9)
+ ROWGATHER_CELLS, ROWGATHER_ROWLIST, ROWGATHER_TASKS) = range(10)
 STRATEGIES = {"atomic": ATOMIC, "coloured": COLOURED, "staged": STAGED, "staged_coloured": STAGED,
               "rowgather": ROWGATHER,
               "rowgather_thread": ROWGATHER_THREAD, "rowgather_slots": ROWGATHER_SLOTS,
               "rowgather_staged": ROWGATHER_STAGED, "rowgather_cells": ROWGATHER_CELLS,
-              "rowgather_rows": ROWGATHER_ROWLIST}
+              "rowgather_rows": ROWGATHER_ROWLIST, "rowgather_tasks": ROWGATHER_TASKS}
 
 _i32p = ctypes.POINTER(ctypes.c_int32)
 
@@ -74,6 +74,10 @@ class ExecPlan(ctypes.Structure):
         ("row_base", ctypes.c_void_p),
         ("subset", ctypes.c_void_p),
         ("batch_packed", ctypes.c_void_p),
+        ("task_desc", ctypes.c_void_p),
+        ("tasks", ctypes.c_void_p),
+        ("task_multis", ctypes.c_void_p),
+        ("max_batch_multis", ctypes.c_int32),
     ]
 
 
@@ -119,6 +123,8 @@ _SIGNATURES = {
     "op2hip_transpose_count_places": (ctypes.c_int, [_I, _V, _I, _I, _V, ctypes.POINTER(ctypes.c_int64),
                                                      _V, _V, ctypes.c_size_t, _V]),
     "op2hip_transpose_fill_places": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, _V]),
+    "op2hip_task_plan_count": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _V]),
+    "op2hip_task_plan_fill": (ctypes.c_int, [_I, _V, _V, _V, _V, _I, _I, _V, _V, _V, _V, _V, _V, _V, _V]),
     "op2hip_mat_slots": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _I, _V, _V, _V]),
     "op2hip_tile_targets_count": (ctypes.c_int, [_I, _I, _V, _I, _V, _V]),
     "op2hip_tile_targets_fill": (ctypes.c_int, [_I, _I, _V, _I, _V, _V, _V, _V]),

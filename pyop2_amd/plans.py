@@ -115,6 +115,7 @@ class RowBatches:
     slots: dict = None   # (cmap id) -> (table, descriptors)
     max_row_nnz: int = None
     cells_plans: dict = None
+    task_plans: dict = None
 
     def exec_fields(self, ex):
         ex.batch_rows = dev.ptr(self.batch_rows)
@@ -163,6 +164,12 @@ class RowBatches:
         more than 255 element blocks (built once)."""
         if len(hit) > 4:
             return hit[4]
+        gt = self._gather_lists(hit, nblocks)
+        key = id(hit[2])
+        self.slots[key] = hit = hit + (gt,)
+        return gt
+
+    def _gather_lists(self, hit, nblocks):
         L = dev.lib()
         table, desc, cmap = hit[0], hit[1], hit[2]
         gcount = dev.empty((max(nblocks, 1),), np.uint8)
@@ -185,9 +192,55 @@ class RowBatches:
                                                      dev.ptr(gcount), dev.ptr(glist), dev.stream()),
                           "gather_table_fill")
                 gt = (gcount, glist)
-        key = id(cmap)
-        self.slots[key] = hit = hit + (gt,)
         return gt
+
+    def task_plan(self, hit, tr, rarity, nblocks):
+        """Task plan (op2hip_task_plan_*) of slot table ``hit``, built once on
+        the device; None when a batch does not fit it."""
+        if self.task_plans is None:
+            self.task_plans = {}
+        cmap = hit[2]
+        if id(cmap) not in self.task_plans:
+            self.task_plans[id(cmap)] = self._make_task_plan(hit, tr, rarity, nblocks)
+        return self.task_plans[id(cmap)]
+
+    def _make_task_plan(self, hit, tr, rarity, nblocks):
+        cmap, nb = hit[2], self.nbatches
+        if self.max_nnz > 1024 or self.max_inc > 1024 or rarity * cmap.arity > 128 or nb == 0:
+            return None
+        gt = self._gather_lists(hit, nblocks)   # in use only until the plan is made
+        if gt is None:
+            return None
+        L, s = dev.lib(), dev.stream()
+        counts = dev.empty((3 * nb + 1,), np.int32)
+        dev.check(L.op2hip_task_plan_count(nb, dev.ptr(hit[1]), dev.ptr(gt[0]), dev.ptr(tr.inc_ent), rarity,
+                                           dev.ptr(counts), s), "task_plan_count")
+        host = dev.to_host(counts)
+        if host[-1]:
+            return None
+        per = host[:-1].reshape(nb, 3).astype(np.int64)
+        first = np.zeros((nb, 3), dtype=np.int64)
+        np.cumsum(per[:-1], axis=0, out=first[1:])
+        total = per.sum(axis=0)
+        if total.max() >= 2 ** 31:
+            return None
+        firsts = [dev.to_device(np.ascontiguousarray(first[:, k], dtype=np.int32)) for k in range(3)]
+        cells = dev.empty((max(int(total[0]), 1),), np.int32)
+        tasks = dev.empty((max(int(total[1]), 1),), np.int32)
+        multis = dev.empty((max(int(total[2]), 1),), np.uint16)
+        desc = dev.empty((nb, 16), np.int32)
+        dev.check(L.op2hip_task_plan_fill(nb, dev.ptr(hit[1]), dev.ptr(gt[0]), dev.ptr(gt[1]),
+                                          dev.ptr(tr.inc_ent), rarity, cmap.arity, *[dev.ptr(f) for f in firsts],
+                                          dev.ptr(cells), dev.ptr(tasks), dev.ptr(multis), dev.ptr(desc), s),
+                  "task_plan_fill")
+        return dict(desc=desc, cells=cells, tasks=tasks, multis=multis,
+                    max_cells=int(per[:, 0].max()), max_multis=int(per[:, 2].max()))
+
+    @staticmethod
+    def task_fields(ex, tp):
+        ex.task_desc, ex.cells = dev.ptr(tp["desc"]), dev.ptr(tp["cells"])
+        ex.tasks, ex.task_multis = dev.ptr(tp["tasks"]), dev.ptr(tp["multis"])
+        ex.max_batch_cells, ex.max_batch_multis = tp["max_cells"], tp["max_multis"]
 
     def cell_gather(self, hit, tr, rarity, nblocks):
         """Cell-gather plan (op2hip_plan_cell_gather) of slot table ``hit``,

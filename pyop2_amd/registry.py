@@ -133,6 +133,15 @@ _BATCH_CELLS = {("p1_laplace_matrix", "f64"): (256, 512),
                 ("p2_elasticity_matrix", "f32"): (256, 512),
                 ("p2_elasticity_fused", "f64"): (256, 512),
                 ("p2_elasticity_fused", "f32"): (256, 512)}
+# The task gather holds a batch's values in their own type, its elements'
+# geometry (112 bytes each), and a lookup table.
+_BATCH_TASKS = (384, 480)
+
+
+def _tasks_lds(max_nnz, max_cells, max_multis, itemsize):
+    return max_nnz * 9 * itemsize + 48 + max_cells * 112 + max_multis * 72 + 16 + 2000
+
+
 _BATCH_STAGED = {("p1_laplace_matrix", "f64"): (256, 512),
                  ("p2_elasticity_matrix", "f64"): (64, 256),
                  ("p2_elasticity_matrix", "f32"): (64, 256),
@@ -257,6 +266,8 @@ class HandWrittenKernel:
             return "atomic"
         if strategy == "split" and "split" not in self.spec:
             return "atomic"
+        if strategy == "rowgather_tasks" and self.family != "p2_elasticity_matrix":
+            strategy = "rowgather_slots"
         if has_mat and strategy.startswith("rowgather"):
             mat = parloop.arguments[0].data
             if mat.block_shape != self.spec["args"][0][2]:
@@ -493,15 +504,28 @@ class HandWrittenKernel:
                     if rb.max_inc > budget[0]:
                         # a row with more incidences than one batch can stage
                         rb, strategy = None, "rowgather_slots"
+                tasks = None
+                if strategy == "rowgather_tasks":
+                    budget = tuple(cfg.get("batch") or _BATCH_TASKS)
+                    rb = plans.row_batches(rmap, tr, mat.rowptr, budget[0], budget[1], key)
+                    hit = rb.slot_table(tr, mat.rowptr, mat.colidx, args[0].maps[1], rmap.arity)
+                    tasks = rb.task_plan(hit, tr, rmap.arity, mat.sparsity.block_nnz) if hit else None
+                    if tasks is None or _tasks_lds(rb.max_nnz, tasks["max_cells"], tasks["max_multis"],
+                                                   mat.dtype.itemsize) > _LDS:
+                        rb, tasks, strategy = None, None, "rowgather_slots"
                 if rb is None:
                     budget = tuple(cfg.get("batch") or _BATCH[(self.family, self.variant)])
                     rb = plans.row_batches(rmap, tr, mat.rowptr, budget[0], budget[1], key)
                 rb.exec_fields(ex)
                 keep.append(rb)
-                if strategy in ("rowgather_slots", "rowgather_staged", "rowgather_cells"):
+                if strategy in ("rowgather_slots", "rowgather_staged", "rowgather_cells", "rowgather_tasks"):
                     hit = rb.slot_table(tr, mat.rowptr, mat.colidx, args[0].maps[1], rmap.arity)
                     if hit is None:
                         strategy = "rowgather_thread"
+                    elif strategy == "rowgather_tasks":
+                        rb.task_fields(ex, tasks)
+                        rb.slot_fields(ex, hit)
+                        keep.append(tasks)
                     elif strategy == "rowgather_cells":
                         cg = rb.cell_gather(hit, tr, rmap.arity, mat.sparsity.block_nnz)
                         if cg is None:
