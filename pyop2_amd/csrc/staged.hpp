@@ -154,26 +154,47 @@ __device__ __forceinline__ void flush_map(const Elem &elem, const TilePlan &P, i
 }
 
 // Second pass of a partials plan: every shared node adds its partials, in
-// tile order, to the Dat (one thread per node; the order of the additions
-// does not depend on scheduling).
+// tile order, to the Dat (one thread per component of a node; the order of
+// the additions does not depend on scheduling).  What bounds it is the chain
+// of a node's loads -- its range, the slots, the partials, the Dat -- with few
+// threads in flight, so the slots and the partials of four tiles (most nodes
+// are shared by fewer) are loaded at once, the Dat's value beside the range,
+// and a node's components lie in neighbouring lanes: 4.6 against 6.6 us at
+// 18 000 nodes of the 32^3 float64 cube; at 665 000 nodes (64^3) the traffic
+// bounds it, 21 us as with a thread per node and one tile's loads at a time.
 template <typename T, int kOut>
 __global__ void __launch_bounds__(256)
 staged_reduce_kernel(int32_t nshared, const int32_t *__restrict__ nodes,
                      const int32_t *__restrict__ ptr, const int32_t *__restrict__ slots,
                      const double *__restrict__ partials, T *__restrict__ out) {
-  const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int kAtOnce = 4;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t s = int32_t(t / kOut), a = int32_t(t % kOut);
   if (s >= nshared) return;
-  double sum[kOut];
+  const int32_t end = ptr[s + 1];
+  int32_t j = ptr[s];
+  T *o = out + (size_t)nodes[s] * kOut + a;
+  const T old = *o;
+  double sum = 0.0;
+  for (; j < end; j += kAtOnce) {
+    int32_t slot[kAtOnce];
+    double v[kAtOnce];
 #pragma unroll
-  for (int a = 0; a < kOut; ++a) sum[a] = 0.0;
-  for (int32_t j = ptr[s]; j < ptr[s + 1]; ++j) {
-    const double *p = partials + (size_t)slots[j] * kOut;
+    for (int u = 0; u < kAtOnce; ++u) slot[u] = slots[j + u < end ? j + u : end - 1];
 #pragma unroll
-    for (int a = 0; a < kOut; ++a) sum[a] += p[a];
+    for (int u = 0; u < kAtOnce; ++u) v[u] = partials[(size_t)slot[u] * kOut + a];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) sum += j + u < end ? v[u] : 0.0;
   }
-  T *o = out + (size_t)nodes[s] * kOut;
-#pragma unroll
-  for (int a = 0; a < kOut; ++a) o[a] = T(double(o[a]) + sum[a]);
+  *o = T(double(old) + sum);
+}
+
+template <typename T, int kOut>
+void launch_staged_reduce(const op2hip_exec *ex, int map, T *out, hipStream_t s) {
+  const int64_t threads = (int64_t)ex->nshared[map] * kOut;
+  staged_reduce_kernel<T, kOut><<<(uint32_t)((threads + 255) / 256), 256, 0, s>>>(
+      ex->nshared[map], ex->shared_nodes[map], ex->shared_ptr[map], ex->shared_slots[map],
+      ex->partials[map], out);
 }
 
 // Whether an element reads its staged values from LDS itself
@@ -358,15 +379,11 @@ int launch_staged(int32_t start, int32_t end, const Elem &elem, const op2hip_exe
   OP2HIP_LAUNCHED();
   if constexpr (Elem::kOut0 > 0) {
     if (P.shared_off[0] && ex->nshared[0] > 0)
-      staged_reduce_kernel<typename Elem::T, Elem::kOut0><<<(ex->nshared[0] + 255) / 256, 256, 0, s>>>(
-          ex->nshared[0], ex->shared_nodes[0], ex->shared_ptr[0], ex->shared_slots[0],
-          ex->partials[0], elem.template out<0>());
+      launch_staged_reduce<typename Elem::T, Elem::kOut0>(ex, 0, elem.template out<0>(), s);
   }
   if constexpr (Elem::kMaps > 1 && Elem::kOut1 > 0) {
     if (P.shared_off[1] && ex->nshared[1] > 0)
-      staged_reduce_kernel<typename Elem::T, Elem::kOut1><<<(ex->nshared[1] + 255) / 256, 256, 0, s>>>(
-          ex->nshared[1], ex->shared_nodes[1], ex->shared_ptr[1], ex->shared_slots[1],
-          ex->partials[1], elem.template out<1>());
+      launch_staged_reduce<typename Elem::T, Elem::kOut1>(ex, 1, elem.template out<1>(), s);
   }
   OP2HIP_LAUNCHED();
   return OP2HIP_OK;
