@@ -799,6 +799,11 @@ struct MatrixLanes {
 template <typename TT>
 struct ResidualStaged {
   using T = TT;
+  // adds each node's increment to the tile's accumulators as it is formed:
+  // 99 against 108 us at 64^3 in float64 (38 against 41 at 45^3 in float32)
+  // with all ten kept to the end.  154 registers, three waves per SIMD; four
+  // waves (128 registers, 25 of them spilled) took 118 us
+  static constexpr bool kLdsScatter = true;
   static constexpr int kMaps = 2;
   static constexpr int kAr0 = 10, kIn0 = 3, kOut0 = 3;
   static constexpr int kAr1 = 4, kIn1 = 3, kOut1 = 0;
@@ -815,9 +820,17 @@ struct ResidualStaged {
   }
   template <int M>
   __host__ __device__ __forceinline__ T *out() const { return R; }
-  __device__ __forceinline__ void element(int32_t, const T (&uu)[10][3], const T (&xv)[4][3],
-                                          T (&re)[10][3], T (&)[4][1]) const {
-    element_residual(uu, geometry_of(xv), lam, mu, re);
+  template <class Add0, class Add1>
+  __device__ __forceinline__ void element_add(int32_t, const T *in0, const uint16_t (&l0)[10],
+                                              const T *in1, const uint16_t (&l1)[4], Add0 &&add0,
+                                              Add1 &&) const {
+    T xv[4][3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) xv[i][a] = in1[3 * l1[i] + a];
+    residual_vertex_form(
+        geometry_of(xv), lam, mu, [&](int j, int c) { return in0[3 * l0[j] + c]; }, add0);
   }
 };
 

@@ -211,6 +211,20 @@ struct LdsElementOf<Elem, std::void_t<decltype(Elem::kLdsElement)>> {
   static constexpr bool value = Elem::kLdsElement;
 };
 
+// Whether an element also adds its contributions to the tile's accumulators
+// itself (Elem::kLdsScatter, with element_add(e, in0, l0, in1, l1, add0,
+// add1): add0(i, v) and add1(i, v) add the array v to local node i).  An
+// element that has each contribution ready for good as it goes keeps no array
+// of all of them live to its end.
+template <class Elem, class = void>
+struct LdsScatterOf {
+  static constexpr bool value = false;
+};
+template <class Elem>
+struct LdsScatterOf<Elem, std::void_t<decltype(Elem::kLdsScatter)>> {
+  static constexpr bool value = Elem::kLdsScatter;
+};
+
 // Tile b of a staged launch (the workgroup's share, or one work item of a
 // batched launch).  The local node ids of a thread's first element are
 // loaded before the staging barrier.
@@ -264,10 +278,23 @@ __device__ __forceinline__ void staged_tile(const Elem &elem, const TilePlan &P,
     const int32_t pos = pos_of(t);
     if (pos >= ne) continue;
     if (t != (int32_t)threadIdx.x) load_locals(p0 + pos);
+    if constexpr (LdsScatterOf<Elem>::value) {
+      elem.element_add(
+          elem_id, in0, l0, in1, l1,
+          [&](int i, const T (&v)[O0]) {
+#pragma unroll
+            for (int a = 0; a < O0; ++a) atomic_add(&acc0[(size_t)l0[i] * O0 + a], double(v[a]));
+          },
+          [&](int i, const T (&v)[O1]) {
+#pragma unroll
+            for (int a = 0; a < O1; ++a) atomic_add(&acc1[(size_t)l1[i] * O1 + a], double(v[a]));
+          });
+      continue;
+    }
     T y0[A0][O0], y1[A1][O1];
     if constexpr (LdsElementOf<Elem>::value) {
       elem.element_lds(elem_id, in0, l0, in1, l1, y0, y1);
-    } else {
+    } else if constexpr (!LdsScatterOf<Elem>::value) {
       T x0[A0][I0], x1[A1][I1];
 #pragma unroll
       for (int i = 0; i < A0; ++i)
