@@ -235,6 +235,11 @@ int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
                      const int32_t *rmap, int32_t rarity, const int32_t *cmap, int32_t carity,
                      int32_t *slots, int32_t *bad, void *stream);
 
+/* *out = half the sum of the squares of n device doubles; partials holds
+ * OP2HIP_HALF_SQUARE_PARTIALS doubles. */
+#define OP2HIP_HALF_SQUARE_PARTIALS 1024
+int op2hip_half_square(int64_t n, const double *x, double *partials, double *out, void *stream);
+
 /* ---- task plan of OP2HIP_ROWGATHER_TASKS -------------------------------- */
 /* From row batches, their slot table's descriptors and a gather table
  * (op2hip_gather_table_*): every output block's element blocks are cut into

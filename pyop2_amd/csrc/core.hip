@@ -651,6 +651,43 @@ __global__ void mat_slots(int64_t total, const int32_t *__restrict__ rowptr,
   }
 }
 
+// Half the sum of squares of n values in two launches: every workgroup writes
+// one partial, the second launch adds them, both in a fixed order.  One pass
+// over memory, where a product, a reduction over it and a scaling were three:
+// 0.8 million values (6.6 MB, from the last-level cache) 4 + 2 against 17 us.
+constexpr int kHalfSquareBlocks = 1024, kHalfSquareAtOnce = 4;
+
+__device__ __forceinline__ double sum_of_workgroup(double v) {
+  __shared__ double waves[16];
+  for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+  if (threadIdx.x % 64 == 0) waves[threadIdx.x / 64] = v;
+  __syncthreads();
+  v = 0.0;
+  for (uint32_t w = 0; w < blockDim.x / 64; ++w) v += waves[w];
+  return v;
+}
+
+__global__ void __launch_bounds__(256)
+half_square_partials(int64_t n, const double *__restrict__ x, double *__restrict__ partials) {
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  double sum = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += stride * kHalfSquareAtOnce) {
+    double v[kHalfSquareAtOnce];
+#pragma unroll
+    for (int u = 0; u < kHalfSquareAtOnce; ++u) v[u] = i + u * stride < n ? x[i + u * stride] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kHalfSquareAtOnce; ++u) sum += v[u] * v[u];
+  }
+  sum = sum_of_workgroup(sum);
+  if (threadIdx.x == 0) partials[blockIdx.x] = sum;
+}
+
+__global__ void __launch_bounds__(kHalfSquareBlocks)
+half_square_total(int32_t n, const double *__restrict__ partials, double *__restrict__ out) {
+  const double sum = sum_of_workgroup((int32_t)threadIdx.x < n ? partials[threadIdx.x] : 0.0);
+  if (threadIdx.x == 0) *out = 0.5 * sum;
+}
+
 __global__ void expand_rowptr(int32_t nrows, const int32_t *__restrict__ rowptr,
                               int32_t rdim, int32_t cdim, int32_t *__restrict__ out) {
   for (int32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= nrows;
@@ -917,6 +954,17 @@ int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
   if (total == 0) return OP2HIP_OK;
   mat_slots<<<std::min<uint32_t>(ceil_div(total, 256), 65536), 256, 0, stream_of(stream)>>>(
       total, rowptr, colidx, rmap, rarity, cmap, carity, slots, bad);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+int op2hip_half_square(int64_t n, const double *x, double *partials, double *out, void *stream) {
+  OP2HIP_REQUIRE(n >= 0 && partials && out && (n == 0 || x), "half_square: bad arguments");
+  hipStream_t s = stream_of(stream);
+  const int32_t grid = (int32_t)std::min<int64_t>((n + 255) / 256, kHalfSquareBlocks);
+  static_assert(kHalfSquareBlocks == OP2HIP_HALF_SQUARE_PARTIALS);
+  if (grid > 0) half_square_partials<<<grid, 256, 0, s>>>(n, x, partials);
+  half_square_total<<<1, kHalfSquareBlocks, 0, s>>>(grid, partials, out);
   OP2HIP_LAUNCHED();
   return OP2HIP_OK;
 }

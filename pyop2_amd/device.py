@@ -125,6 +125,7 @@ _SIGNATURES = {
     "op2hip_transpose_fill_places": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, _V]),
     "op2hip_task_plan_count": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _V]),
     "op2hip_task_plan_fill": (ctypes.c_int, [_I, _V, _V, _V, _V, _I, _I, _V, _V, _V, _V, _V, _V, _V, _V]),
+    "op2hip_half_square": (ctypes.c_int, [ctypes.c_int64, _V, _V, _V, _V]),
     "op2hip_mat_slots": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _I, _V, _V, _V]),
     "op2hip_tile_targets_count": (ctypes.c_int, [_I, _I, _V, _I, _V, _V]),
     "op2hip_tile_targets_fill": (ctypes.c_int, [_I, _I, _V, _I, _V, _V, _V, _V]),

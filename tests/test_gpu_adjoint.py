@@ -118,3 +118,32 @@ def test_gradient_against_cpu_tangent_linear(device):
         tlm = float((Rh * dR).sum())
         ad = float((u.grad.cpu().numpy() * du).sum() + (x.grad.cpu().numpy() * dX).sum())
         assert abs(tlm - ad) <= 1e-11 * abs(tlm)
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 257, 1023, 262144, 262145, 1048577, 3000001])
+def test_half_square(device, n):
+    """One value to many per thread, partials from none to all.  The sum of n
+    squares in any order is within n eps of exact; in blocks as here far
+    closer: 1e-13."""
+    x = np.random.default_rng(n).standard_normal(n)
+    R = dev.to_device(x)
+    want = 0.5 * np.dot(x.astype(np.longdouble), x.astype(np.longdouble))
+    for _ in range(2):
+        J = adjoint._half_square(R)
+        assert J.shape == () and abs(float(J) - want) <= 1e-13 * abs(want)
+
+
+def test_objective_is_the_residuals_half_square(device, problem32):
+    """Value, both gradients and a factor on the way back, against the same
+    expression of the differentiable residual: rounding of sums of 1e6 terms
+    and of values from atomics-free loops, 1e-12."""
+    m, p, prob, X, rng = problem32
+    got = []
+    for f in (prob.objective, lambda u, x: 0.5 * (prob.residual(u, x) ** 2).sum()):
+        u = p.u.device_data_ro.clone().requires_grad_(True)
+        x = p.X.device_data_ro.clone().requires_grad_(True)
+        J = f(u, x)
+        (3.0 * J).backward()
+        got.append([dev.to_host(t.detach()) for t in (J.reshape(1), u.grad, x.grad)])
+    for a, b in zip(*got):
+        assert relerr(a, b) < 1e-12
