@@ -630,11 +630,23 @@ tile_targets_add(int32_t nrows, int32_t dim, const int32_t *__restrict__ ptr,
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)nrows * dim) return;
   const int32_t r = dim == 1 ? (int32_t)i : (int32_t)(i / dim), j = (int32_t)(i - (int64_t)r * dim);
-  const int32_t lo = ptr[r], hi = ptr[r + 1];
-  if (lo == hi) return;
+  constexpr int kAtOnce = 2;
+  int32_t k = ptr[r];
+  const int32_t end = ptr[r + 1];
+  if (k == end) return;
+  const T old = out[i];
   A sum = A(0);
-  for (int32_t k = lo; k < hi; ++k) sum += partials[(int64_t)slots[k] * dim + j];
-  out[i] = T(A(out[i]) + sum);
+  for (; k < end; k += kAtOnce) {
+    int32_t slot[kAtOnce];
+    A v[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) slot[u] = slots[k + u < end ? k + u : end - 1];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) v[u] = partials[(int64_t)slot[u] * dim + j];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) sum += k + u < end ? v[u] : A(0);
+  }
+  out[i] = T(A(old) + sum);
 }
 
 __global__ void mat_slots(int64_t total, const int32_t *__restrict__ rowptr,
