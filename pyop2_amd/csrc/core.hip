@@ -663,6 +663,36 @@ __global__ void mat_slots(int64_t total, const int32_t *__restrict__ rowptr,
   }
 }
 
+// Smallest and largest of n entries: a pair per workgroup, bound by one read of
+// the entries.
+__global__ void __launch_bounds__(256)
+entry_range(int64_t n, const int32_t *__restrict__ v, int32_t *__restrict__ pairs) {
+  __shared__ int32_t least[4], most[4];
+  int32_t lo = INT32_MAX, hi = INT32_MIN;
+#pragma unroll 4
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    lo = min(lo, v[i]);
+    hi = max(hi, v[i]);
+  }
+  for (int d = 32; d > 0; d >>= 1) {
+    lo = min(lo, __shfl_xor(lo, d));
+    hi = max(hi, __shfl_xor(hi, d));
+  }
+  if (threadIdx.x % 64 == 0) {
+    least[threadIdx.x / 64] = lo;
+    most[threadIdx.x / 64] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) {
+      lo = min(lo, least[w]);
+      hi = max(hi, most[w]);
+    }
+    pairs[2 * blockIdx.x] = lo;
+    pairs[2 * blockIdx.x + 1] = hi;
+  }
+}
+
 // Half the sum of squares of n values in two launches: every workgroup writes
 // one partial, the second launch adds them, both in a fixed order.  One pass
 // over memory, where a product, a reduction over it and a scaling were three:
@@ -966,6 +996,14 @@ int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
   if (total == 0) return OP2HIP_OK;
   mat_slots<<<std::min<uint32_t>(ceil_div(total, 256), 65536), 256, 0, stream_of(stream)>>>(
       total, rowptr, colidx, rmap, rarity, cmap, carity, slots, bad);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+int op2hip_entry_range(int64_t n, const int32_t *values, int32_t npairs, int32_t *pairs,
+                       void *stream) {
+  OP2HIP_REQUIRE(n >= 0 && npairs > 0 && pairs && (n == 0 || values), "entry_range: bad arguments");
+  entry_range<<<npairs, 256, 0, stream_of(stream)>>>(n, values, pairs);
   OP2HIP_LAUNCHED();
   return OP2HIP_OK;
 }

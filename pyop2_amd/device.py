@@ -125,6 +125,7 @@ _SIGNATURES = {
     "op2hip_transpose_fill_places": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, _V]),
     "op2hip_task_plan_count": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _V]),
     "op2hip_task_plan_fill": (ctypes.c_int, [_I, _V, _V, _V, _V, _I, _I, _V, _V, _V, _V, _V, _V, _V, _V]),
+    "op2hip_entry_range": (ctypes.c_int, [ctypes.c_int64, _V, _I, _V, _V]),
     "op2hip_half_square": (ctypes.c_int, [ctypes.c_int64, _V, _V, _V, _V]),
     "op2hip_mat_slots": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _I, _V, _V, _V]),
     "op2hip_tile_targets_count": (ctypes.c_int, [_I, _I, _V, _I, _V, _V]),
@@ -319,6 +320,14 @@ def to_device(a):
         src = t.from_numpy(a.view(view))
         return src.to(dev).view(torch_dtype(a.dtype))
     return t.from_numpy(a).to(dev)
+
+
+def entry_range(values):
+    """Smallest and largest entry of a device int32 tensor that has some."""
+    pairs = empty((256, 2), np.int32)
+    check(lib().op2hip_entry_range(values.numel(), ptr(values), 256, ptr(pairs), stream()), "entry_range")
+    h = to_host(pairs)
+    return int(h[:, 0].min()), int(h[:, 1].max())
 
 
 def to_host(tensor, out=None):

@@ -11,6 +11,11 @@ from pyop2_amd import exceptions as ex, utils
 from pyop2_amd.datatypes import IntType
 from pyop2_amd.types.set import Set
 
+# Least entries whose range is found on the device, in one launch and one copy
+# back (26 us), rather than by two passes of a host core (19 us for 0.26, 33 for
+# 0.52, 50 for 0.83, 131 us for 2.1 million entries)
+_RANGE_ON_DEVICE = 1 << 19
+
 
 class Map:
 
@@ -164,10 +169,16 @@ class Map:
         if self._dev is None:
             from pyop2_amd import device as dev
             v = np.ascontiguousarray(self._table, dtype=IntType)
-            self._has_negative = bool(v.size and v.min() < 0)
-            if v.size and v.max() >= self._toset.total_size:
+            t, (lo, hi) = None, (0, -1)
+            if v.size >= _RANGE_ON_DEVICE:
+                t = dev.to_device(v)
+                lo, hi = dev.entry_range(t)
+            elif v.size:
+                lo, hi = int(v.min()), int(v.max())
+            self._has_negative = lo < 0
+            if hi >= self._toset.total_size:
                 raise ex.MapValueError(f"{self} has entries >= {self._toset.total_size} (target set size)")
-            self._dev = dev.to_device(v)
+            self._dev = dev.to_device(v) if t is None else t
         return self._dev
 
     @property
