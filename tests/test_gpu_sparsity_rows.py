@@ -76,3 +76,41 @@ def test_incidences_ascend(device, nrows, ncells):
     order = np.argsort(t.ravel(), kind="stable")
     assert np.array_equal(dev.to_host(tr.inc_ptr), np.searchsorted(t.ravel()[order], np.arange(nrows + 1)))
     assert np.array_equal(dev.to_host(tr.inc_ent)[:tr.total], order)
+
+
+@pytest.mark.parametrize("n", [0, 1, 7, 2048, 2049, 300000, 1024 * 2048, 1024 * 2048 + 1, 2500000])
+def test_exclusive_scan(device, n):
+    """One tile, several, the most whose sums the blocks take themselves, more."""
+    import ctypes
+    v = np.random.default_rng(n).integers(0, 7, n).astype(np.int32)
+    t, out = dev.to_device(v), dev.empty((n + 1,), np.int32)
+    L, need, total = dev.lib(), ctypes.c_size_t(), ctypes.c_int64()
+    dev.check(L.op2hip_scan_workspace(n, ctypes.byref(need)))
+    work = dev.empty((need.value,), np.uint8)
+    for _ in range(2):
+        dev.check(L.op2hip_exclusive_scan(n, dev.ptr(t), dev.ptr(out), ctypes.byref(total), dev.ptr(work),
+                                          need.value, dev.stream()))
+        want = np.concatenate(([0], np.cumsum(v)))
+        assert total.value == want[-1] and np.array_equal(dev.to_host(out), want)
+
+
+@pytest.mark.parametrize("nrows", [1, 64, 65, 5000])
+def test_entries_beyond_the_set_are_counted(device, nrows):
+    """The counter lies behind the counts, whatever their number."""
+    import ctypes
+    v = np.random.default_rng(1).integers(0, nrows, (900, 3)).astype(np.int32)
+    L, need, total = dev.lib(), ctypes.c_size_t(), ctypes.c_int64()
+    dev.check(L.op2hip_transpose_workspace(nrows, ctypes.byref(need)))
+    work, ptr = dev.empty((need.value,), np.uint8), dev.empty((nrows + 1,), np.int32)
+
+    def count():
+        return L.op2hip_transpose_count(nrows, dev.ptr(t), 3, 900, dev.ptr(ptr), ctypes.byref(total),
+                                        dev.ptr(work), need.value, dev.stream())
+    t = dev.to_device(v)
+    dev.check(count())
+    assert total.value == v.size
+    assert np.array_equal(np.diff(dev.to_host(ptr)), np.bincount(v.ravel(), minlength=nrows))
+    v[5, 1] = v[899, 2] = nrows
+    t = dev.to_device(v)
+    with pytest.raises(dev.DeviceError, match="2 map entries"):
+        dev.check(count())
