@@ -21,7 +21,7 @@ semantics (``pyop2/codegen/builder.py``):
 
 Indirect WRITE/RW arguments and Mat WRITE need exclusive targets, so such
 loops run coloured (greedy colouring, one launch per colour); INC-only
-loops run with atomics, or in tiles (``_Tiling``): a workgroup adds the
+loops run with atomics, or in tiles (``_tiles``): a workgroup adds the
 increments of consecutive elements up in LDS, writes one partial sum per
 distinct target, and a second pass adds a target's partial sums.  Sources
 are compiled for gfx950 with hiprtc and the code objects cached in memory

@@ -653,9 +653,11 @@ tile_targets(int32_t n, int32_t tile, const int32_t *__restrict__ table, int32_t
 }
 
 // Partial sums of every target, one thread per target and component: bound by
-// its scattered 8-byte reads (11 us for 361,201 targets of four values, 14 us
-// for the 1,753,001 entries of a P1 matrix; the tiles before it take 24 and 11
-// us, where device atomics took 72 and 137 us).
+// its scattered 8-byte reads, so two slots and their partials are loaded at
+// once and the output's value beside the range (10 us for 361,201 targets of
+// four values, 13 us for the 1,753,001 entries of a P1 matrix, 11 and 14.5 us
+// one at a time; the tiles before it take 24 and 11 us, where device atomics
+// took 72 and 137 us).
 template <typename T, typename A>
 __global__ void __launch_bounds__(256)
 tile_targets_add(int32_t nrows, int32_t dim, const int32_t *__restrict__ ptr,

@@ -22,7 +22,9 @@
 //   void element(int32_t e, const T (&x0)[A0][I0], const T (&x1)[A1][I1],
 //                T (&y0)[A0][O0], T (&y1)[A1][O1]) const;     // A/I/O >= 1
 //   or, with kLdsElement = true, element_lds(e, in0, l0, in1, l1, y0, y1)
-//   reading the staged records from LDS itself (see LdsElementOf).
+//   reading the staged records from LDS itself (see LdsElementOf), or, with
+//   kLdsScatter = true, element_add(e, in0, l0, in1, l1, add0, add1) adding
+//   its increments itself as well (see LdsScatterOf).
 #pragma once
 
 #include "launch.hpp"
@@ -159,9 +161,10 @@ __device__ __forceinline__ void flush_map(const Elem &elem, const TilePlan &P, i
 // of a node's loads -- its range, the slots, the partials, the Dat -- with few
 // threads in flight, so the slots and the partials of four tiles (most nodes
 // are shared by fewer) are loaded at once, the Dat's value beside the range,
-// and a node's components lie in neighbouring lanes: 4.6 against 6.6 us at
-// 18 000 nodes of the 32^3 float64 cube; at 665 000 nodes (64^3) the traffic
-// bounds it, 21 us as with a thread per node and one tile's loads at a time.
+// and a node's components lie in neighbouring lanes: the three passes of a
+// gradient on the 32^3 float64 cube (residual, and the adjoint's nodes and
+// vertices) take 4.6 us on average, 6.6 with a thread per node and one tile's
+// loads at a time; at 665,000 nodes (64^3) the traffic bounds it, 21 us each way.
 template <typename T, int kOut>
 __global__ void __launch_bounds__(256)
 staged_reduce_kernel(int32_t nshared, const int32_t *__restrict__ nodes,
