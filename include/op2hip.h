@@ -235,6 +235,8 @@ int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
                      const int32_t *rmap, int32_t rarity, const int32_t *cmap, int32_t carity,
                      int32_t *slots, int32_t *bad, void *stream);
 
+/* Zero `bytes` bytes of device memory that starts on a 16-byte boundary. */
+int op2hip_clear(void *data, int64_t bytes, void *stream);
 /* Smallest and largest of n entries in npairs pairs (INT32_MAX, INT32_MIN for
  * none), whose own smallest and largest are the entries'. */
 int op2hip_entry_range(int64_t n, const int32_t *values, int32_t npairs, int32_t *pairs,

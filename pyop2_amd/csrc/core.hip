@@ -699,6 +699,29 @@ __global__ void mat_slots(int64_t total, const int32_t *__restrict__ rowptr,
   }
 }
 
+// Zero bytes from a 16-byte boundary on, bound by the stores.  Four words a
+// thread; beyond the 256 MB of the last-level cache one word a thread, stored
+// past the caches.  A pass with the loop that follows, against torch's fill:
+// 23 MB 25.1 and 26.5 us, 52 MB 104.5 and 108, 59 MB 96 and 99; 765 MB 576 and
+// 597 (four plain words a thread 599; past the caches, 52 MB would take 110).
+typedef uint32_t ClearWord __attribute__((ext_vector_type(4)));
+constexpr int64_t kClearCached = 256ll << 20;
+
+template <int kWords, bool kPast>
+__global__ void __launch_bounds__(256)
+clear_words(ClearWord *__restrict__ p, int64_t n, uint8_t *__restrict__ rest, int32_t nrest) {
+  const int64_t first = (int64_t)blockIdx.x * (256 * kWords) + threadIdx.x;
+  const ClearWord zero = {0, 0, 0, 0};
+#pragma unroll
+  for (int u = 0; u < kWords; ++u) {
+    const int64_t i = first + u * 256;
+    if (i >= n) break;
+    if (kPast) __builtin_nontemporal_store(zero, p + i);
+    else p[i] = zero;
+  }
+  if (first < nrest) rest[first] = 0;
+}
+
 // Smallest and largest of n entries: a pair per workgroup, bound by one read of
 // the entries.
 __global__ void __launch_bounds__(256)
@@ -1029,6 +1052,23 @@ int op2hip_mat_slots(int32_t n, const int32_t *rowptr, const int32_t *colidx,
   if (total == 0) return OP2HIP_OK;
   mat_slots<<<std::min<uint32_t>(ceil_div(total, 256), 65536), 256, 0, stream_of(stream)>>>(
       total, rowptr, colidx, rmap, rarity, cmap, carity, slots, bad);
+  OP2HIP_LAUNCHED();
+  return OP2HIP_OK;
+}
+
+int op2hip_clear(void *data, int64_t bytes, void *stream) {
+  OP2HIP_REQUIRE(bytes >= 0 && (bytes == 0 || (data && reinterpret_cast<uintptr_t>(data) % 16 == 0)),
+                 "clear: bad arguments");
+  if (bytes == 0) return OP2HIP_OK;
+  hipStream_t s = stream_of(stream);
+  const int64_t n = bytes / 16;
+  ClearWord *p = static_cast<ClearWord *>(data);
+  uint8_t *rest = reinterpret_cast<uint8_t *>(p + n);
+  const int32_t nrest = (int32_t)(bytes % 16);
+  if (bytes > kClearCached)
+    clear_words<1, true><<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(p, n, rest, nrest);
+  else
+    clear_words<4, false><<<(uint32_t)std::max<int64_t>(1, (n + 1023) / 1024), 256, 0, s>>>(p, n, rest, nrest);
   OP2HIP_LAUNCHED();
   return OP2HIP_OK;
 }

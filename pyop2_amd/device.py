@@ -125,6 +125,7 @@ _SIGNATURES = {
     "op2hip_transpose_fill_places": (ctypes.c_int, [_I, _V, _I, _I, _V, _V, _V, _V]),
     "op2hip_task_plan_count": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _V]),
     "op2hip_task_plan_fill": (ctypes.c_int, [_I, _V, _V, _V, _V, _I, _I, _V, _V, _V, _V, _V, _V, _V, _V]),
+    "op2hip_clear": (ctypes.c_int, [_V, ctypes.c_int64, _V]),
     "op2hip_entry_range": (ctypes.c_int, [ctypes.c_int64, _V, _I, _V, _V]),
     "op2hip_half_square": (ctypes.c_int, [ctypes.c_int64, _V, _V, _V, _V]),
     "op2hip_mat_slots": (ctypes.c_int, [_I, _V, _V, _V, _I, _V, _I, _V, _V, _V]),
@@ -320,6 +321,22 @@ def to_device(a):
         src = t.from_numpy(a.view(view))
         return src.to(dev).view(torch_dtype(a.dtype))
     return t.from_numpy(a).to(dev)
+
+
+def clear(t):
+    """``t.zero_()``, by a kernel of the library where it takes the tensor:
+    whole, on the op2 device, from a 16-byte boundary on, and without the
+    autograd state that zero_ has to look at.  The tensor's version counts
+    the write either way."""
+    at = t.data_ptr()
+    if (at % 16 or not t.is_contiguous() or t.get_device() != configuration["device"] or t.requires_grad
+            or t.is_inference()):
+        t.zero_()
+        return
+    rc = lib().op2hip_clear(at, t.nbytes, raw_stream())
+    if rc:
+        check(rc, "clear")
+    torch().autograd.graph.increment_version(t)
 
 
 def entry_range(values):

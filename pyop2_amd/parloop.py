@@ -27,6 +27,7 @@ argument, again under the reference's names (``DatLegacyArg`` ...).
 """
 import numpy as np
 
+from pyop2_amd import device as dev
 from pyop2_amd.configuration import configuration
 from pyop2_amd.exceptions import KernelTypeError, MapValueError, SetTypeError
 from pyop2_amd.global_kernel import (DatKernelArg, GlobalKernel, GlobalKernelArg, MatKernelArg,
@@ -294,7 +295,7 @@ class Parloop:
         for target in versioned:
             target.increment_dat_version()
         for tmp in self.reduced_globals:
-            tmp._device_array().zero_()
+            dev.clear(tmp._device_array())
             tmp._device_modified()
         for mat, state in mats:
             mat.change_assembly_state(state)
@@ -341,7 +342,6 @@ class Parloop:
 
 
 def _signed_of(t):
-    from pyop2_amd import device as dev
     torch = dev.torch()
     return {1: torch.int8, 2: torch.int16, 4: torch.int32, 8: torch.int64}[t.element_size()]
 

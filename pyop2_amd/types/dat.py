@@ -10,7 +10,7 @@ import contextlib
 
 import numpy as np
 
-from pyop2_amd import configuration as conf, exceptions as ex, utils
+from pyop2_amd import configuration as conf, device as dev, exceptions as ex, utils
 from pyop2_amd.types.access import Access
 from pyop2_amd.types.data_carrier import DataCarrier, DeviceStorage
 from pyop2_amd.types.dataset import DataSet
@@ -46,7 +46,6 @@ class AbstractDat(DataCarrier, DeviceStorage):
 
     @property
     def _kernel_args_(self):
-        from pyop2_amd import device as dev
         return (dev.ptr(self._device_array()),)
 
     @utils.validate_in(('access', _modes, ex.ModeValueError))
@@ -166,7 +165,7 @@ class AbstractDat(DataCarrier, DeviceStorage):
             self.data[self._owned_rows_of(subset)] = 0
             return
         if self._device_current():
-            self._device_array().zero_()
+            dev.clear(self._device_array())
             self._device_modified()
         else:
             self._host_array().fill(0)

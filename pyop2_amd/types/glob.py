@@ -8,7 +8,7 @@ import numbers
 
 import numpy as np
 
-from pyop2_amd import exceptions as ex, utils
+from pyop2_amd import device as dev, exceptions as ex, utils
 from pyop2_amd.types.access import Access
 from pyop2_amd.types.data_carrier import DataCarrier, DeviceStorage
 
@@ -25,7 +25,6 @@ class SetFreeDataCarrier(DataCarrier, DeviceStorage):
 
     @property
     def _kernel_args_(self):
-        from pyop2_amd import device as dev
         return (dev.ptr(self._device_array()),)
 
     def __iter__(self):
@@ -213,7 +212,7 @@ class Global(SetFreeDataCarrier):
         assert subset is None
         self.increment_dat_version()
         if self._where in (2, 3):
-            self._device_array().zero_()
+            dev.clear(self._device_array())
             self._device_modified()
         else:
             self._host_array()[...] = 0

@@ -565,8 +565,9 @@ class Mat(DataCarrier):
 
     def zero(self):
         """Zero every stored value (the pattern is kept)."""
+        from pyop2_amd import device as dev
         self._init()
-        self._values.zero_()
+        dev.clear(self._values)
 
     # -- entries set from the host (the reference's MatSetValues calls) ----------
     # A few entries change on the device; only their positions are found on
